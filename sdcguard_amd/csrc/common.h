@@ -179,6 +179,39 @@ __device__ __forceinline__ int64_t wave_max_i64_dpp(int64_t v) {
   return r;
 }
 
+// The worst keys of a check's result row (res[0]: key, res[1]: key with its noise; both hold the score's bits in
+// their high half), raised by one thread of a workgroup.  Device-scope maxima on one address from every XCD
+// serialize at about 14 ns each: on a row that starts at zero, as every queued check's does, two for each of a
+// pass's thousands of workgroups took longer than the pass (fp8 4096 x 14336: 227 us; the linear check's pass over
+// y: 100 us).  So a workgroup first raises a slot that only its own XCD uses (the line stays in that XCD's L2; the
+// slots are cleared by a kernel earlier in the call: sdc_clear_slots), and goes on to the row only with a key that
+// was the slot's largest so far, about ln(workgroups / 8) times a slot: 41 us and 35 us (32 slots picked by the
+// workgroup's number: 73 and 54 us).  The largest key of all is the largest of its slot whenever it comes, so it
+// always reaches the row, whichever slots the workgroups took.  A lower score than the slot's cannot raise either
+// word.  seen0, seen1: the row's keys read earlier (keys only grow: a stale value only lets a maximum through).
+constexpr int SDC_SLOTS = 8;                                             // one per XCD
+constexpr int SDC_SLOT_WORDS = 16;                                       // 128 bytes each
+constexpr int SDC_SLOT_FLOATS = SDC_SLOTS * SDC_SLOT_WORDS * 2;          // workspace of a set of slots, in floats
+__device__ __forceinline__ void sdc_raise_worst(int64_t* res, unsigned long long* slots, int64_t key, int64_t keyd,
+                                                int64_t seen0, int64_t seen1) {
+  if (key <= seen0 && keyd <= seen1) return;
+  const uint32_t xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11));        // HW_REG_XCC_ID, bits 0 .. 3
+  unsigned long long* s = slots + SDC_SLOT_WORDS * (xcc % SDC_SLOTS);
+  const unsigned long long k0 = (unsigned long long)key, k1 = (unsigned long long)keyd;
+  const unsigned long long o0 = atomicMax(s, k0);
+  if ((k0 >> 32) < (o0 >> 32)) return;
+  const unsigned long long o1 = atomicMax(s + 1, k1);
+  if (k0 > o0 && key > seen0) atomicMax((unsigned long long*)res, k0);
+  if (k1 > o1 && keyd > seen1) atomicMax((unsigned long long*)(res + 1), k1);
+}
+// (called by every thread of one workgroup of an earlier kernel; `sets` sets of slots, null: none)
+__device__ __forceinline__ void sdc_clear_slots(unsigned long long* slots, int sets, int t, int threads) {
+  if (slots) {
+    for (int i = t; i < sets * SDC_SLOTS * SDC_SLOT_WORDS; i += threads) slots[i] = 0ull;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (the GEMMs count their own loads from here on)
+  }
+}
+
 // bits of a float as an int64 holding the unsigned 32-bit pattern
 __device__ __forceinline__ int64_t fbits64(float f) { return (int64_t)(uint32_t)__float_as_uint(f); }
 

@@ -33,6 +33,9 @@ struct GemmArgs {
   // (the tall-tile kernel, an fp8 A) 64-row tiles instead of 128, for a short A whose 128-row tiles would leave
   // most CUs idle
   int short_rows;
+  // sets of result slots that workgroup 0 clears for the scoring pass that follows (null: none)
+  unsigned long long* slots;
+  int slot_sets;
 };
 
 // E and XN for `batches` batches.

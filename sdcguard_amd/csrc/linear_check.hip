@@ -283,6 +283,7 @@ struct YArgs {
   const uint16_t* bias;            // (n) or null
   int64_t* result;                 // int64[3]: key, key with noise, unjudged
   float* zrow;                     // (n, mb, 2) scores or null
+  unsigned long long* slots;       // result slots of the column check, then of the row check (sdc_raise_worst)
   // constants of both noise models
   float u, h, abs_floor, l1c, zt, lim_a, lim_big, capk;
 };
@@ -592,8 +593,7 @@ __global__ __launch_bounds__(256) void ypass_kernel(YArgs a) {
     const int64_t d0 = red_d[w0] > red_d[w0 + 1] ? red_d[w0] : red_d[w0 + 1];
     const int un = red_u[w0] + red_u[w0 + 1];
     int64_t* res = t == 0 ? a.state : a.result;
-    if (k0 > seen0) atomicMax((unsigned long long*)res, (unsigned long long)k0);
-    if (d0 > seen1) atomicMax((unsigned long long*)(res + 1), (unsigned long long)d0);
+    sdc_raise_worst(res, a.slots + (t == 0 ? 0 : SDC_SLOTS * SDC_SLOT_WORDS), k0, d0, seen0, seen1);
     if (t == 0) {
       if (blockIdx.x == 0 && blockIdx.y == 0) atomicAdd((unsigned long long*)(res + 2), 1ull);
       if (un > 0) atomicAdd((unsigned long long*)(res + 3), (unsigned long long)un);
@@ -606,7 +606,7 @@ __global__ __launch_bounds__(256) void ypass_kernel(YArgs a) {
 struct Layout {
   int64_t nb, mb, rem_n, rem_m, nkc, kp, scol, srow;
   bool rs_col, rs_row, tall_col, tall_row;
-  int64_t off_parts, off_stats, off_xnp, off_xn, off_rstat, off_erow, off_ecol, off_fcol, total;   // in floats
+  int64_t off_parts, off_stats, off_xnp, off_xn, off_rstat, off_erow, off_ecol, off_fcol, off_slots, total;   // in floats
 };
 
 Layout layout(int64_t m, int64_t k, int64_t n) {
@@ -639,6 +639,7 @@ Layout layout(int64_t m, int64_t k, int64_t n) {
   L.off_ecol = o; o += al(L.scol * 2 * L.nb * m);
   // (the layer's parts in fragment order, made here when the caller passes none)
   L.off_fcol = o; o += L.rs_col ? al(sdc_parts_fragments_bytes(2 * L.nb, k) / 4) : 0;
+  L.off_slots = o; o += 2 * SDC_SLOT_FLOATS;
   L.total = o;
   return L;
 }
@@ -701,6 +702,7 @@ int queue_both(const void* x, int64_t sxm, const void* W, int64_t swn, const voi
   gc.m = m; gc.k = k; gc.N = 2 * L.nb; gc.splits = L.scol;
   gc.E = ws + L.off_ecol; gc.XN = nullptr; gc.et = 1;
   gc.prof_name = "col_gemm";
+  gc.slots = (unsigned long long*)(ws + L.off_slots); gc.slot_sets = 2;
   int rc = SDC_EUNSUPPORTED;
   if (L.rs_col && (parts_frag ||
                    sdc_parts_fragments(parts, spc, 2 * L.nb, k, ws + L.off_fcol, side) == SDC_OK)) {
@@ -768,6 +770,7 @@ int queue_both(const void* x, int64_t sxm, const void* W, int64_t swn, const voi
   ya.state = state; ya.zcol = col_scores;
   ya.Erow = ws + L.off_erow; ya.wn = w_norms; ya.srow = gr.splits; ya.rstat = ws + L.off_rstat;
   ya.bias = (const uint16_t*)bias; ya.result = row_result; ya.zrow = row_scores;
+  ya.slots = gc.slots;
   ya.u = 1.f / 256.f; ya.h = 0.f; ya.abs_floor = abs_floor;
   ya.l1c = (float)(k * 7.450580596923828e-09 > 1e-5 ? k * 7.450580596923828e-09 : 1e-5);   // checksum.py:95-104
   ya.zt = z; ya.lim_a = 1e18f; ya.lim_big = 1e18f;

@@ -36,6 +36,7 @@ struct QuantArgs {
   float unit, per_out, zt;
   int c_bf16;
   int64_t* result;                   // [4]: worst key, key with its noise, wrong blocks, blocks with non-finite values
+  unsigned long long* slots;         // the result slots, cleared by the GEMM (sdc_raise_worst)
   float* zdump;                      // (m, nb) z per block, or null
 };
 
@@ -236,8 +237,7 @@ __global__ __launch_bounds__(256) void quant_score_kernel(QuantArgs a) {
     }
     int64_t* res = a.result;
     const int64_t s0 = __atomic_load_n(res, __ATOMIC_RELAXED), s1 = __atomic_load_n(res + 1, __ATOMIC_RELAXED);
-    if (k0 > s0) atomicMax((unsigned long long*)res, (unsigned long long)k0);
-    if (d0 > s1) atomicMax((unsigned long long*)(res + 1), (unsigned long long)d0);
+    sdc_raise_worst(res, a.slots, k0, d0, s0, s1);
     if (wsum > 0) atomicAdd((unsigned long long*)(res + 2), (unsigned long long)wsum);
     if (nsum > 0) atomicAdd((unsigned long long*)(res + 3), (unsigned long long)nsum);
   }
@@ -514,8 +514,7 @@ __global__ __launch_bounds__(256) void quant_tile_kernel(QuantArgs a) {
     const int wr = wave_sum_i32_dpp(best.wrong), nf = wave_sum_i32_dpp(best.nonfin);
     if (lane == 0) {
       int64_t* res = a.result;
-      if (key > seen0) atomicMax((unsigned long long*)res, (unsigned long long)key);
-      if (keyd > seen1) atomicMax((unsigned long long*)(res + 1), (unsigned long long)keyd);
+      sdc_raise_worst(res, a.slots, key, keyd, seen0, seen1);
       if (wr > 0) atomicAdd((unsigned long long*)(res + 2), (unsigned long long)wr);
       if (nf > 0) atomicAdd((unsigned long long*)(res + 3), (unsigned long long)nf);
     }
@@ -538,7 +537,7 @@ int64_t quant_splits(int kind, int64_t m, int64_t k, int64_t ncols) {
 }
 
 struct QLayout {
-  int64_t nb, rem, ncols, splits, nacc, kpad, off_e, off_xn, off_apad, off_ppad, off_frag, total;   // in floats
+  int64_t nb, rem, ncols, splits, nacc, kpad, off_e, off_xn, off_apad, off_ppad, off_frag, off_slots, total;   // in floats
   bool tall;                       // the tall-tile register-streamed GEMM where the shape allows
   bool short_rows;                 // (its 64-row tiles, for a short A)
   int64_t tsplits;                 // (its depth parts: planes of E)
@@ -580,6 +579,7 @@ QLayout qlayout(int kind, int64_t m, int64_t k, int64_t n, int64_t bs) {
   L.off_ppad = o; o += al(sdc_cdiv(2 * L.ncols * L.kpad, 4));
   L.off_frag = o;
   o += L.tall ? al((kind == 0 ? sdc_digit_fragments_bytes(L.ncols, k) : sdc_parts_fragments_bytes(L.ncols, k)) / 4) : 0;
+  L.off_slots = o; o += SDC_SLOT_FLOATS;
   L.total = o;
   return L;
 }
@@ -670,6 +670,7 @@ extern "C" int sdc_quant_check(int kind, const void* A, int64_t sam, const void*
   g.m = m; g.k = kg; g.N = L.ncols; g.splits = L.splits;
   g.E = ws + L.off_e; g.XN = ws + L.off_xn;
   g.prof_name = kind == 0 ? "quant_gemm_i8" : "quant_gemm_fp8";
+  g.slots = (unsigned long long*)(ws + L.off_slots); g.slot_sets = 1;
   int rc = SDC_EUNSUPPORTED;
   int64_t splits = L.splits;
   if (L.tall && tiles && sam % 16 == 0 && (uintptr_t)A % 16 == 0 && spc % 8 == 0 && spc >= k &&
@@ -708,7 +709,7 @@ extern "C" int sdc_quant_check(int kind, const void* A, int64_t sam, const void*
   qa.per_out = (float)(sqrt((double)k) + (nfma > 0.f ? (double)k / (double)nfma : 0.0));
   qa.zt = z;
   qa.c_bf16 = c_dtype == C_BF16;
-  qa.result = result; qa.zdump = scores_out;
+  qa.result = result; qa.slots = g.slots; qa.zdump = scores_out;
   SdcProf prof(kind == 0 ? "quant_score_i8" : "quant_score_fp8", stream);
   if (tiles) {
     // bf16 C: 128-row tiles (32 KB; measured 13% faster than 64 rows at 4096 x 14336); 4-byte C
