@@ -776,8 +776,8 @@ __global__ __launch_bounds__(64 * RS_WAVES, 1) void rs_gemm_kernel(GemmArgs g) {
 constexpr int GSCAN = 1024;                       // groups the grouped tall GEMM takes
 
 // TCF: 32-column fragments a tile (2; 1 for outputs of at most 32 columns, whose second fragment would be empty)
-template <int DT, int ROLE, int TRF, int AT, bool XNORM, bool GROUPED = false, int TCF = 2>
-__global__ __launch_bounds__(64 * RS_WAVES, TRF == 4 ? 1 : 2) void rs_gemm_tall_kernel(GemmArgs g) {
+template <int DT, int ROLE, int TRF, int AT, bool XNORM, bool GROUPED = false, int TCF = 2, int NW = RS_WAVES>
+__global__ __launch_bounds__(64 * NW, TRF == 4 ? 1 : 2) void rs_gemm_tall_kernel(GemmArgs g) {
   constexpr int MDT = AT ? SDC_BF16 : DT;       // the MFMAs' type (AT 2: int8)
   constexpr int SPS = AT ? 8 : 4;               // steps per segment
   constexpr int SD = 16 * SPS;                  // depths per segment
@@ -788,14 +788,15 @@ __global__ __launch_bounds__(64 * RS_WAVES, TRF == 4 ? 1 : 2) void rs_gemm_tall_
   static_assert(AT != 2 || (TRF == 2 && !XNORM && !GROUPED), "int8: 64-row tiles, no row norms");
   static_assert(TCF == 1 || TCF == 2, "one or two column fragments a tile");
   constexpr int TR = 32 * TRF, TC = 32 * TCF, RB = 4, NAI = TR / 8, APS = NAI / SPS;
+  static_assert(TR % (4 * NW) == 0 && TC % (NW * (256 / TR)) == 0, "the epilogue's shares of rows and columns");
   constexpr int RT_SEGB = TR * 128;             // bytes of A per wave and segment (TR rows x 128 bytes)
-  constexpr int RED_BYTES = RS_WAVES * TC * (TR + 4) * 4;       // the epilogue's reduction (below)
+  constexpr int RED_BYTES = NW * TC * (TR + 4) * 4;       // the epilogue's reduction (below)
   __shared__ __attribute__((aligned(16)))
-  uint8_t smem[RS_WAVES * 2 * RT_SEGB > RED_BYTES ? RS_WAVES * 2 * RT_SEGB : RED_BYTES];
-  __shared__ float xred[XNORM ? RS_WAVES : 1][XNORM ? TR : 1][2];
+  uint8_t smem[NW * 2 * RT_SEGB > RED_BYTES ? NW * 2 * RT_SEGB : RED_BYTES];
+  __shared__ float xred[XNORM ? NW : 1][XNORM ? TR : 1][2];
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, 64 * RS_WAVES);
+  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, 64 * NW);
   const int r = lane & 31, h = lane >> 5;
   const int64_t N = g.N, m = g.m;
   // (tile indices in 32 bits, their divisions by run-time divisors the short unsigned ones: the launcher keeps the
@@ -815,7 +816,7 @@ __global__ __launch_bounds__(64 * RS_WAVES, TRF == 4 ? 1 : 2) void rs_gemm_tall_
     // the grid covers (ceil(m / TR) + groups) row tiles per column tile and half -- workgroups past the last exit
     __shared__ int64_t gend[GSCAN], gtile[GSCAN];
     const int ng = (int)g.ngroups;
-    for (int q = t; q < ng; q += 64 * RS_WAVES) {
+    for (int q = t; q < ng; q += 64 * NW) {
       const int64_t e = min(max(g.goffs[q], (int64_t)0), m), s0 = q ? min(max(g.goffs[q - 1], (int64_t)0), m) : 0;
       gend[q] = e;
       gtile[q] = e > s0 ? sdc_cdiv(e - s0, TR) : 0;
@@ -864,8 +865,10 @@ __global__ __launch_bounds__(64 * RS_WAVES, TRF == 4 ? 1 : 2) void rs_gemm_tall_
   const uint32_t ct = tile % nct;
   const int64_t c0 = (int64_t)ct * TC;
   const bool do_xn = XNORM && ct == 0;
-  const int per = (int)((uint32_t)(g.k / SD) / (uint32_t)(RS_WAVES * g.splits));   // segments per wave
-  const int seg0 = (int)half * per * RS_WAVES + w * per;
+  // the depth's segments dealt to the NW waves of every depth part in order, as evenly as they go
+  const uint32_t nseg = (uint32_t)(g.k / SD), slot = half * NW + (uint32_t)w, slots = NW * (uint32_t)g.splits;
+  const int seg0 = (int)(nseg * slot / slots);
+  const int per = (int)(nseg * (slot + 1) / slots) - seg0;      // segments of this wave (0: more waves than segments)
   uint8_t* const abuf = smem + w * 2 * RT_SEGB;
   // LDS address of fragment i (rows 32 i + r) at step jj of a segment: the 16-bit depth piece 4 h + jj, or the
   // fp8 byte offset 64 (jj / 4) + 32 h + 8 (jj % 4) (its 16-byte chunk c, swizzled by the row, and half of it)
@@ -1025,9 +1028,12 @@ __global__ __launch_bounds__(64 * RS_WAVES, TRF == 4 ? 1 : 2) void rs_gemm_tall_
           SDC_TALL_WAIT_B((RB - 1) * (APS + NP * TCF), sl);
         }
         if constexpr (TRF == 4)
-          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fr[cur][0]), "+v"(fr[cur][1]), "+v"(fr[cur][2]), "+v"(fr[cur][3]));
+          asm volatile("s_waitcnt lgkmcnt(0)"
+                       : "+v"(fr[cur][0]), "+v"(fr[cur][TRF > 1]), "+v"(fr[cur][TRF / 2]), "+v"(fr[cur][TRF - 1]));
+        else if constexpr (TRF == 2)
+          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fr[cur][0]), "+v"(fr[cur][TRF - 1]));
         else
-          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fr[cur][0]), "+v"(fr[cur][1]));
+          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fr[cur][0]));
         AOpT a[TRF];
 #pragma unroll
         for (int i = 0; i < TRF; ++i) {
@@ -1104,7 +1110,7 @@ __global__ __launch_bounds__(64 * RS_WAVES, TRF == 4 ? 1 : 2) void rs_gemm_tall_
     if (do_xn && t < TR) {
       float sq = xred[0][t][0], ab = xred[0][t][1];
 #pragma unroll
-      for (int q = 1; q < RS_WAVES; ++q) {
+      for (int q = 1; q < NW; ++q) {
         sq += xred[q][t][0];
         ab += xred[q][t][1];
       }
@@ -1119,8 +1125,8 @@ __global__ __launch_bounds__(64 * RS_WAVES, TRF == 4 ? 1 : 2) void rs_gemm_tall_
   // wave's 16-byte writes spread over the banks) and are added in wave (depth) order; each store instruction then
   // writes two whole columns of the tile (2 x TR floats, contiguous in the transposed plane).
   constexpr int RP = TR + 4;
-  float* red = reinterpret_cast<float*>(smem);                  // [RS_WAVES][TC][RP]
-  static_assert(RS_WAVES * TC * RP * 4 <= (int)sizeof(smem), "the reduction fits the shared memory");
+  float* red = reinterpret_cast<float*>(smem);                  // [NW][TC][RP]
+  static_assert(NW * TC * RP * 4 <= (int)sizeof(smem), "the reduction fits the shared memory");
   const int64_t me = g.m;
   constexpr int LPC = TR / 4;                                   // lanes per column (4 rows each)
   constexpr int CPI = 64 / LPC;                                 // columns per store instruction
@@ -1147,14 +1153,14 @@ __global__ __launch_bounds__(64 * RS_WAVES, TRF == 4 ? 1 : 2) void rs_gemm_tall_
       // wave order, as below)
       const int c4 = 4 * (lane & 15);
 #pragma unroll
-      for (int gq = 0; gq < TR / 16; ++gq) {
-        const int rl = w * (TR / 4) + 4 * gq + (lane >> 4);
+      for (int gq = 0; gq < TR / (4 * NW); ++gq) {
+        const int rl = w * (TR / NW) + 4 * gq + (lane >> 4);
         f32x4 v;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float x = red[(c4 + e) * RP + rl];
 #pragma unroll
-          for (int q = 1; q < RS_WAVES; ++q) {
+          for (int q = 1; q < NW; ++q) {
             const float u = red[(q * TC + c4 + e) * RP + rl];
             if constexpr (AT == 2) x = __int_as_float(__float_as_int(x) + __float_as_int(u));
             else x += u;
@@ -1177,11 +1183,11 @@ __global__ __launch_bounds__(64 * RS_WAVES, TRF == 4 ? 1 : 2) void rs_gemm_tall_
     }
     }
 #pragma unroll
-    for (int gq = 0; gq < TC / (RS_WAVES * CPI); ++gq) {
-      const int cl = (w * (TC / (RS_WAVES * CPI)) + gq) * CPI + lc;   // the tile's column
+    for (int gq = 0; gq < TC / (NW * CPI); ++gq) {
+      const int cl = (w * (TC / (NW * CPI)) + gq) * CPI + lc;   // the tile's column
       f32x4 v = *reinterpret_cast<const f32x4*>(red + cl * RP + 4 * lr);
 #pragma unroll
-      for (int q = 1; q < RS_WAVES; ++q) {
+      for (int q = 1; q < NW; ++q) {
         const f32x4 u = *reinterpret_cast<const f32x4*>(red + (q * TC + cl) * RP + 4 * lr);
         if constexpr (AT == 2)
           v = __builtin_bit_cast(f32x4, __builtin_bit_cast(i32x4, v) + __builtin_bit_cast(i32x4, u));
@@ -1272,24 +1278,52 @@ int sdc_rs_gemm_launch(int dtype, GemmArgs g, int role, hipStream_t stream) {
   return SDC_OK;
 }
 
-// The tall-tile variant: 128 x 64 tiles (64 x 64 with g.short_rows, fp8 only) over g.splits (1 .. SDC_MAX_SPLITS)
-// depth parts, one plane of E per part (the depth a multiple of 256 splits, of 512 splits for an fp8 A; A's rows
-// 16-byte aligned); with g.XN set, also A's row norms, one plane per part.  dtype SDC_FP8: an fp8 e4m3 A widened to bf16 (B's parts bf16).  With g.goffs (16-bit A
-// only): rows grouped by the groups' cumulative ends, group q's fragments at g.B + q g.sbb, row norms always.
-// Returns SDC_EUNSUPPORTED where it does not apply.
+// Row tiles (32, 64 or 128 rows) and depth parts of the tall-tile GEMM for 16-bit rows, m x k against N columns: the
+// shortest tile that holds a short m whole (16 rows against 128-row tiles multiply seven eighths padding), then the
+// number of parts, at most SDC_MAX_SPLITS, with the least rounds of 256 workgroups x (set-up + a wave's segments) +
+// the planes' traffic.  The set-up (about 6 us: the first loads and the epilogue), a segment's time (1.6 us for 128
+// rows, 0.7 us for 32) and 5 TB/s for a plane written and read back are this GEMM's as measured on MI355X.
+TallPlan sdc_tall_plan(int64_t m, int64_t k, int64_t N) {
+  TallPlan p{0, 0};
+  if (m < 1 || N < 1 || k < 64 || k % 64) return p;
+  p.short_rows = m <= 32 ? 2 : m <= 64 ? 1 : 0;
+  const int64_t tr = 128 >> p.short_rows, nw = p.short_rows ? 8 : RS_WAVES, nseg = k / 64;
+  const int64_t tiles = sdc_cdiv(m, tr) * sdc_cdiv(N, 64);
+  const double seg = 0.4 + 1.2 * (double)tr / 128.0, plane = 8e-6 * (double)m * (double)N / 5.0;
+  double best = 0.0;
+  for (int64_t s = 1; s <= SDC_MAX_SPLITS && s * nw <= nseg + nw - 1; ++s) {
+    const double c = (double)sdc_cdiv(tiles * s, 256) * (6.0 + seg * (double)sdc_cdiv(nseg, nw * s)) + plane * (double)s;
+    if (p.splits == 0 || c < best) {
+      p.splits = s;
+      best = c;
+    }
+  }
+  return p;
+}
+
+// The tall-tile variant: 128 x 64 tiles (g.short_rows 1 or 2: 64 x 64 or 32 x 64; for a 16-bit A only with g.XN and
+// no groups) over g.splits (1 .. SDC_MAX_SPLITS) depth parts, one plane of E per part (the depth a multiple of 64, of
+// 128 for a byte A, dealt to the parts' waves in whole segments; A's rows 16-byte aligned); with g.XN set, also A's
+// row norms, one plane per part.  dtype SDC_FP8: an fp8 e4m3 A widened to bf16 (B's parts bf16).  With g.goffs
+// (16-bit A only): rows grouped by the groups' cumulative ends, group q's fragments at g.B + q g.sbb, row norms
+// always.  Returns SDC_EUNSUPPORTED where it does not apply.
 int sdc_rs_gemm_tall_launch(int dtype, GemmArgs g, int role, hipStream_t stream) {
   if (dtype != SDC_BF16 && dtype != SDC_FP16 && dtype != SDC_FP8 && dtype != SDC_I8) return SDC_EUNSUPPORTED;
   const bool byte_a = dtype == SDC_FP8 || dtype == SDC_I8;
-  const int64_t es = byte_a ? 1 : 2, kmul = (byte_a ? RS_WAVES * 128 : RS_KMULT) * g.splits;
-  if (g.splits < 1 || g.splits > SDC_MAX_SPLITS || g.sak != 1 || g.k % kmul || (g.sam * es) % 16 ||
+  const int64_t es = byte_a ? 1 : 2, kmul = byte_a ? 128 : 64;
+  if (g.splits < 1 || g.splits > SDC_MAX_SPLITS || g.sak != 1 || g.k < kmul || g.k % kmul ||
+      g.k / kmul > 0xFFFFFF || (g.sam * es) % 16 ||
       ((uintptr_t)g.A | (uintptr_t)g.B) % 16 || (!g.et && (g.goffs || ((uintptr_t)g.E % 16))))
     return SDC_EUNSUPPORTED;
   if (g.goffs && (dtype == SDC_FP8 || g.ngroups < 1 || g.ngroups > GSCAN || g.sbb % 8)) return SDC_EUNSUPPORTED;
   if (g.m < 1 || g.N < 1) return SDC_EINVAL;
-  if ((g.short_rows || dtype == SDC_I8) && (!byte_a || g.goffs || g.xf_blocks || (dtype == SDC_I8 && g.XN)))
+  if ((g.short_rows || dtype == SDC_I8) && (g.goffs || g.xf_blocks || (dtype == SDC_I8 && g.XN)))
+    return SDC_EUNSUPPORTED;
+  if (g.short_rows < 0 || g.short_rows > (byte_a ? 1 : 2) || (g.short_rows && !byte_a && !g.XN))
     return SDC_EUNSUPPORTED;
   if (dtype == SDC_I8) g.short_rows = 1;                        // (int8: 64-row tiles only)
-  const int64_t rtiles = sdc_cdiv(g.m, g.short_rows ? 64 : 32 * SDC_TALL_TRF) + (g.goffs ? g.ngroups : 0);
+  const int64_t tr = g.short_rows == 2 ? 32 : g.short_rows ? 64 : 32 * SDC_TALL_TRF;
+  const int64_t rtiles = sdc_cdiv(g.m, tr) + (g.goffs ? g.ngroups : 0);
   if (g.xf_blocks < 0 || (g.xf_blocks && (g.goffs || dtype == SDC_FP8))) return SDC_EINVAL;
   // (grouped outputs of at most 32 columns: one-fragment tiles, whose grid counts 32-column tiles)
   const bool narrow = g.goffs && g.N <= 32;
@@ -1316,6 +1350,17 @@ int sdc_rs_gemm_tall_launch(int dtype, GemmArgs g, int role, hipStream_t stream)
   } else if (dtype == SDC_FP8) {
     if (g.XN) hipLaunchKernelGGL((rs_gemm_tall_kernel<SDC_BF16, 3, T, 1, true>), grid, block, 0, stream, g);
     else hipLaunchKernelGGL((rs_gemm_tall_kernel<SDC_BF16, 3, T, 1, false>), grid, block, 0, stream, g);
+  } else if (g.short_rows) {
+    // (a short 16-bit A: eight waves a workgroup, each an eighth of its part's depth)
+    const dim3 b8(64 * 8);
+    if (g.short_rows == 2 && dtype == SDC_BF16)
+      hipLaunchKernelGGL((rs_gemm_tall_kernel<SDC_BF16, 6, 1, 0, true, false, 2, 8>), grid, b8, 0, stream, g);
+    else if (g.short_rows == 2)
+      hipLaunchKernelGGL((rs_gemm_tall_kernel<SDC_FP16, 6, 1, 0, true, false, 2, 8>), grid, b8, 0, stream, g);
+    else if (dtype == SDC_BF16)
+      hipLaunchKernelGGL((rs_gemm_tall_kernel<SDC_BF16, 6, 2, 0, true, false, 2, 8>), grid, b8, 0, stream, g);
+    else
+      hipLaunchKernelGGL((rs_gemm_tall_kernel<SDC_FP16, 6, 2, 0, true, false, 2, 8>), grid, b8, 0, stream, g);
   } else if (role == 1) {
     if (dtype == SDC_BF16) hipLaunchKernelGGL((rs_gemm_tall_kernel<SDC_BF16, 1, T, 0, false>), grid, block, 0, stream, g);
     else hipLaunchKernelGGL((rs_gemm_tall_kernel<SDC_FP16, 1, T, 0, false>), grid, block, 0, stream, g);

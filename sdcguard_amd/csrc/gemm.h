@@ -30,8 +30,8 @@ struct GemmArgs {
   // for them
   XStageArgs xf;
   int xf_blocks;
-  // (the tall-tile kernel, an fp8 A) 64-row tiles instead of 128, for a short A whose 128-row tiles would leave
-  // most CUs idle
+  // (the tall-tile kernel) 1: 64-row tiles instead of 128, 2: 32-row tiles (16-bit A only), for a short A whose
+  // 128-row tiles would be mostly padding or leave most CUs idle
   int short_rows;
   // sets of result slots that workgroup 0 clears for the scoring pass that follows (null: none)
   unsigned long long* slots;
@@ -46,6 +46,11 @@ int sdc_gemm_launch(int dtype, GemmArgs g, int64_t batches, hipStream_t stream);
 // SDC_EUNSUPPORTED, launching nothing, where their shape or alignment rules do not hold.
 int sdc_rs_gemm_launch(int dtype, GemmArgs g, int role, hipStream_t stream);
 int sdc_rs_gemm_tall_launch(int dtype, GemmArgs g, int role, hipStream_t stream);
+struct TallPlan {
+  int64_t splits;               // depth parts (0: the tall-tile GEMM does not take this depth)
+  int short_rows;
+};
+TallPlan sdc_tall_plan(int64_t m, int64_t k, int64_t N);
 extern "C" int64_t sdc_expected_splits(int64_t m, int64_t k, int64_t ncols);
 extern "C" int64_t sdc_parts_fragments_bytes(int64_t N, int64_t k);
 extern "C" int sdc_parts_fragments(const void* parts, int64_t spc, int64_t N, int64_t k, void* out, hipStream_t stream);

@@ -243,10 +243,16 @@ __global__ __launch_bounds__(256) void serve_pairs_kernel(ScoreArgs a, const flo
 
 }  // namespace
 
+// Planes of E and of x's row norms in the workspace: the staged GEMM's, or the tall-tile GEMM's where it has more.
+static int64_t serve_planes(int64_t m, int64_t k, int64_t ncols) {
+  const int64_t s = sdc_expected_splits(m, k, ncols), t = sdc_tall_plan(m, k, ncols).splits;
+  return s > t ? s : t;
+}
+
 extern "C" int64_t sdc_check_static_workspace(int64_t m, int64_t k, int64_t n, int64_t bs) {
   if (m <= 0 || n <= 0 || bs <= 0) return 0;
   const int64_t nb = sdc_cdiv(n, bs), ncols = 2 * nb;
-  const int64_t splits = sdc_expected_splits(m, k, ncols);
+  const int64_t splits = serve_planes(m, k, ncols);
   // E planes, row-norm planes, then the (4, m * nb) pair sums of the split design
   return (splits * m * ncols + splits * 2 * m + 4 * m * nb) * (int64_t)sizeof(float) + 512;
 }
@@ -274,8 +280,9 @@ extern "C" int sdc_check_static(int dtype, const void* x, int64_t sxm, int64_t s
   const int64_t nb = sdc_cdiv(n, bs), rem = n % bs, ncols = 2 * nb;
   const int64_t splits = sdc_expected_splits(m, k, ncols);
   float* E = (float*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
-  float* XN = E + splits * m * ncols;
-  float* SUMS = (float*)(((uintptr_t)(XN + splits * 2 * m) + 255) & ~(uintptr_t)255);
+  const int64_t planes = serve_planes(m, k, ncols);
+  float* XN = E + planes * m * ncols;
+  float* SUMS = (float*)(((uintptr_t)(XN + planes * 2 * m) + 255) & ~(uintptr_t)255);
   // (the fused persistent pass measured fastest at every batch size on MI355X; v3 stays available on request)
   const bool split_design = kernel == 3 || kernel == 4;
   const double u = dtype == SDC_BF16 ? 1.0 / 256.0 : 1.0 / 2048.0;
@@ -304,19 +311,23 @@ extern "C" int sdc_check_static(int dtype, const void* x, int64_t sxm, int64_t s
   a.vec = (syn == 1) && (sym % 8 == 0) && (bs % 8 == 0) && ((uintptr_t)y % 16 == 0);
   a.yv.vec = a.vec;
   if (cap_meta && (!cap_data || cap_w < bs)) return SDC_EINVAL;
-  // The expected side: the register-streamed tall-tile GEMM (two depth halves, row-major planes, x's row norms in
-  // the same pass) where the parts come in fragment order and the shape suits it, else the staged GEMM
+  // The expected side: the register-streamed tall-tile GEMM (row-major planes, x's row norms in the same pass) where
+  // the parts come in fragment order (a depth of whole 64s), else the staged GEMM.  The staged GEMM's tiles leave
+  // most of the chip idle at a decode step (16 rows: one 256- or 512-row tile a column tile, 8 to 40 workgroups) and
+  // for narrow outputs.  Measured at 16 rows, staged and tall: 3584 deep x 56 columns 24 and 8.5 us, x 592 columns
+  // 23 and 8.7 us, 18944 deep x 56 98 and 16 us; at 4096 rows: 3584 x 56 33 and 18 us, 18944 x 56 123 and
+  // 44 us.
   auto expected = [&]() -> int {
-    if (parts_frag && nparts == 3 && spk == 1 && sxk == 1 && splits >= 2 && k % 512 == 0 &&
-        2 * sdc_cdiv(m, 128) * sdc_cdiv(ncols, 64) >= 192) {
+    const TallPlan plan = sdc_tall_plan(m, k, ncols);
+    if (parts_frag && nparts == 3 && spk == 1 && sxk == 1 && plan.splits > 0) {
       GemmArgs g{};
       g.A = (const uint16_t*)x; g.sam = sxm; g.sak = 1;
-      g.B = parts_frag; g.m = m; g.k = k; g.N = ncols; g.splits = 2;
+      g.B = parts_frag; g.m = m; g.k = k; g.N = ncols; g.splits = plan.splits; g.short_rows = plan.short_rows;
       g.E = E; g.XN = XN; g.et = 0;
       g.prof_name = "expected_gemm";
       const int rc = sdc_rs_gemm_tall_launch(dtype, g, 0, stream);
       if (rc != SDC_EUNSUPPORTED) {
-        a.splits = 2;
+        a.splits = plan.splits;
         return rc;
       }
     }

@@ -80,8 +80,8 @@ def check_linear_both(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torc
 def _fragments(P: torch.Tensor, ncols: int, k: int) -> Optional[torch.Tensor]:
     """The layer's parts in the register-streamed GEMM's fragment order (sdc_parts_fragments), made once and kept on
     the parts tensor (so they live as long as the constants they copy); None where that GEMM does not apply (depth
-    not a multiple of 256, part columns not 16-byte aligned)."""
-    if k % 256 or P.stride(1) % 8 or P.data_ptr() % 16:
+    not a multiple of 64, part columns not 16-byte aligned)."""
+    if k % 64 or P.stride(1) % 8 or P.data_ptr() % 16:
         return None
     key = (P.data_ptr(), P._version, ncols, k)
     hit = getattr(P, "_sdc_frag", None)

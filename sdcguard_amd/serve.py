@@ -217,7 +217,7 @@ def check_static_impl(x2: torch.Tensor, y2: torch.Tensor, parts: torch.Tensor, p
     L = _lib.lib()
     # the parts in fragment order for the tall-tile GEMM (made once, kept on the parts tensor), where it applies
     frag = None
-    if k % 512 == 0 and x2.stride(1) == 1 and x2.data_ptr() % 16 == 0 and (x2.stride(0) * x2.element_size()) % 16 == 0:
+    if k % 64 == 0 and x2.stride(1) == 1 and x2.data_ptr() % 16 == 0 and (x2.stride(0) * x2.element_size()) % 16 == 0:
         from .linear import _fragments
         frag = _fragments(P, 2 * nb, k)
     ws_bytes = int(L.sdc_check_static_workspace(m, k, n, bs))
