@@ -15,6 +15,7 @@
 #include "gemm.h"
 #include "mfma_pipe.h"
 #include "profile.h"
+#include "split.h"
 
 namespace {
 
@@ -50,15 +51,6 @@ __device__ __forceinline__ u32x4 fp8x8_to_bf16(u32x2 v) {
   return o;
 }
 
-// a . b + c over the two 16-bit halves of a and b (fp32 accumulation)
-template <int DT>
-__device__ __forceinline__ float pk_dot2(uint32_t a, uint32_t b, float c) {
-  if constexpr (DT == SDC_BF16)
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
-  else
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b), c, false);
-}
-
 // 8 consecutive (in depth) 16-bit elements at p[kk * sk], or zeros past `lim`
 template <bool VEC>
 __device__ __forceinline__ u32x4 load8(const uint16_t* p, int64_t sk, int64_t kk, int64_t lim, bool ok) {
@@ -90,46 +82,6 @@ __device__ __forceinline__ u32x4 load8_fp8(const uint8_t* p, int64_t sk, int64_t
     pv[i / 2] = lo | (hi << 16);
   }
   return v;
-}
-
-__device__ __forceinline__ uint32_t to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (u >> 16) | 0x40u;       // NaN stays NaN (quiet)
-  u += 0x7FFFu + ((u >> 16) & 1u);                                    // round to nearest even
-  return u >> 16;
-}
-
-template <int DT>
-__device__ __forceinline__ uint32_t round_bits(float f) {
-  if constexpr (DT == SDC_BF16) return to_bf16_bits(f);
-  else return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)f);
-}
-
-template <int DT>
-__device__ __forceinline__ float bits_value(uint32_t b) {
-  return half_to_f32<DT>((uint16_t)b);
-}
-
-// fp32 -> hi, mid, lo parts of 8 values (checksum._split3), packed as three u32x4
-template <int DT>
-__device__ __forceinline__ void split8(const float* v, u32x4* parts) {
-  uint32_t h[8], md[8], lo[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    h[i] = round_bits<DT>(v[i]);
-    const float r = v[i] - bits_value<DT>(h[i]);
-    md[i] = round_bits<DT>(r);
-    lo[i] = round_bits<DT>(r - bits_value<DT>(md[i]));
-  }
-  uint32_t* o0 = reinterpret_cast<uint32_t*>(&parts[0]);
-  uint32_t* o1 = reinterpret_cast<uint32_t*>(&parts[1]);
-  uint32_t* o2 = reinterpret_cast<uint32_t*>(&parts[2]);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    o0[i] = h[2 * i] | (h[2 * i + 1] << 16);
-    o1[i] = md[2 * i] | (md[2 * i + 1] << 16);
-    o2[i] = lo[2 * i] | (lo[2 * i + 1] << 16);
-  }
 }
 
 template <int DT>
@@ -1283,10 +1235,10 @@ int sdc_rs_gemm_launch(int dtype, GemmArgs g, int role, hipStream_t stream) {
 // number of parts, at most SDC_MAX_SPLITS, with the least rounds of 256 workgroups x (set-up + a wave's segments) +
 // the planes' traffic.  The set-up (about 6 us: the first loads and the epilogue), a segment's time (1.6 us for 128
 // rows, 0.7 us for 32) and 5 TB/s for a plane written and read back are this GEMM's as measured on MI355X.
-TallPlan sdc_tall_plan(int64_t m, int64_t k, int64_t N) {
+TallPlan sdc_tall_plan(int64_t m, int64_t k, int64_t N, bool short_ok) {
   TallPlan p{0, 0};
   if (m < 1 || N < 1 || k < 64 || k % 64) return p;
-  p.short_rows = m <= 32 ? 2 : m <= 64 ? 1 : 0;
+  p.short_rows = !short_ok ? 0 : m <= 32 ? 2 : m <= 64 ? 1 : 0;
   const int64_t tr = 128 >> p.short_rows, nw = p.short_rows ? 8 : RS_WAVES, nseg = k / 64;
   const int64_t tiles = sdc_cdiv(m, tr) * sdc_cdiv(N, 64);
   const double seg = 0.4 + 1.2 * (double)tr / 128.0, plane = 8e-6 * (double)m * (double)N / 5.0;

@@ -46,11 +46,13 @@ int sdc_gemm_launch(int dtype, GemmArgs g, int64_t batches, hipStream_t stream);
 // SDC_EUNSUPPORTED, launching nothing, where their shape or alignment rules do not hold.
 int sdc_rs_gemm_launch(int dtype, GemmArgs g, int role, hipStream_t stream);
 int sdc_rs_gemm_tall_launch(int dtype, GemmArgs g, int role, hipStream_t stream);
+// The same product for an A of any alignment, with unit depth stride or unit row stride (lane_gemm.hip)
+int sdc_lane_gemm_launch(int dtype, GemmArgs g, hipStream_t stream);
 struct TallPlan {
   int64_t splits;               // depth parts (0: the tall-tile GEMM does not take this depth)
   int short_rows;
 };
-TallPlan sdc_tall_plan(int64_t m, int64_t k, int64_t N);
+TallPlan sdc_tall_plan(int64_t m, int64_t k, int64_t N, bool short_ok);
 extern "C" int64_t sdc_expected_splits(int64_t m, int64_t k, int64_t ncols);
 extern "C" int64_t sdc_parts_fragments_bytes(int64_t N, int64_t k);
 extern "C" int sdc_parts_fragments(const void* parts, int64_t spc, int64_t N, int64_t k, void* out, hipStream_t stream);

@@ -1,0 +1,319 @@
+// Expected side E = A @ (three parts of the block sums) for an A that the whole-line GEMMs cannot stream: rows that are
+// contiguous across each other (a weight gradient's dy^T: element (row, kk) at A[kk * sak + row]), or rows whose
+// starts are not 16-byte aligned or whose depth is not whole 64s (an output head of 50257 columns).
+//
+// As in the tall-tile GEMM, a workgroup of 4 waves owns a 128 x 64 tile of E over one depth part, each wave a share
+// of that part's 64-deep segments, and the parts of B come in fragment order (zero past the depth); the waves' sums
+// meet in LDS at the end.  A goes from global memory straight into the MFMA operands' registers, four 16-deep steps
+// ahead, which needs no alignment (global loads take any 2-byte address) and no LDS:
+//   rows contiguous: lane (r, h) reads rows 4 r .. 4 r + 3 (8 bytes) at the eight depths 32 h + 8 j .. + 7 of step j,
+//     256 contiguous bytes an instruction and half wave; four v_perm pairs per row turn the eight depths x four rows
+//     into four fragments, fragment i holding rows 4 r + i (which rows a fragment holds is free: the epilogue knows);
+//   depth contiguous: lane (r, h) reads 16 bytes of row 32 i + r at depths 32 h + 8 j, so the four steps of a segment
+//     take the two halves of its 128 bytes.
+// Bound by the latency its four steps in flight cover (16 KB a wave, one workgroup a CU) and the matrix cores.
+// Measured on MI355X against the staged GEMM's element loads: dy^T 14336 x 4096 34 us, from 125 us; dy 1024 x
+// 50257 203 us, from 1267 us; dy^T 50257 x 1024 69 us, from 111 us.
+#include "common.h"
+#include "gemm.h"
+#include "mfma_pipe.h"
+#include "profile.h"
+#include "split.h"
+
+namespace {
+
+constexpr int NW = 4, TRF = 4, TCF = 2, TR = 128, TC = 64, RP = TR + 4;
+
+typedef u32x2 __attribute__((aligned(2))) u32x2_any;        // 8 and 16 bytes at any 2-byte address
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+
+// ROWS: rows contiguous (g.sam 1, g.sak >= g.m >= 4); else depth contiguous (g.sak 1)
+template <int DT, bool ROWS>
+__global__ __launch_bounds__(64 * NW, 1) void lane_gemm_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) float red[NW * TC * RP];
+  __shared__ float xred[NW][TR][2];
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, 64 * NW);
+  const int64_t m = g.m, k = g.k, N = g.N;
+  const uint32_t nct = ((uint32_t)N + TC - 1) / TC, ncf = ((uint32_t)N + 31) / 32;
+  const uint32_t tiles = (uint32_t)((m + TR - 1) / TR) * nct;
+  const uint32_t G = gridDim.x, b = blockIdx.x;
+  const uint32_t wid = (G % 8 == 0) ? (b % 8) * (G / 8) + b / 8 : b;       // XCD x: the x-th eighth of the tiles
+  const uint32_t part = wid / tiles, tile = wid - part * tiles, ct = tile % nct;
+  const int64_t r0 = (int64_t)(tile / nct) * TR, c0 = (int64_t)ct * TC;
+  const bool do_xn = ct == 0 && g.XN != nullptr;
+  // this wave's segments; the last segment of the depth goes through guarded loads where it is not whole, or (rows
+  // contiguous) where a lane's four rows may run past the last row: at every earlier depth those bytes are the next
+  // depth's first rows (sak >= m), and the rows of E they feed are never stored
+  const uint32_t nseg = (uint32_t)((k + 63) / 64), slot = part * NW + (uint32_t)w, slots = NW * (uint32_t)g.splits;
+  const int seg0 = (int)((uint64_t)nseg * slot / slots), seg1 = (int)((uint64_t)nseg * (slot + 1) / slots);
+  const bool guard_last = (k % 64) != 0 || (ROWS && (m % 4) != 0);
+  const bool tail = guard_last && seg1 == (int)nseg && seg1 > seg0;
+  const int nf = seg1 - seg0 - (tail ? 1 : 0);                              // segments read without guards
+
+  const uint16_t* A = g.A;
+  const uint16_t* ap[ROWS ? 1 : TRF];
+  if constexpr (ROWS) {
+    const int64_t row = r0 + 4 * r;
+    ap[0] = A + (row < m ? row : m - 4) + (64 * (int64_t)seg0 + 32 * h) * g.sak;
+  } else {
+#pragma unroll
+    for (int i = 0; i < TRF; ++i) {
+      const int64_t row = r0 + 32 * i + r;
+      ap[i] = A + (row < m ? row : m - 1) * g.sam + 64 * (int64_t)seg0 + 32 * h;
+    }
+  }
+  const int64_t bstep = 3 * (int64_t)ncf * 512;
+  const uint16_t* bq = (const uint16_t*)g.B + 4 * (int64_t)seg0 * bstep + 8 * lane;
+  int bf[TCF];
+#pragma unroll
+  for (int n = 0; n < TCF; ++n) {
+    const uint32_t f = (uint32_t)(c0 / 32) + n;
+    bf[n] = (int)((f < ncf ? f : ncf - 1) * 512);
+  }
+
+  uint32_t ra[4][16];                       // steps in flight: eight depths x 8 bytes, or four rows x 16 bytes
+  u32x4 rb[4][3][TCF];
+  auto load_a = [&](int j, int sg) {        // step j of this wave's segment sg
+    if constexpr (ROWS) {
+      const uint16_t* p = ap[0] + (64 * (int64_t)sg + 8 * j) * g.sak;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const u32x2 v = *reinterpret_cast<const u32x2_any*>(p + e * g.sak);
+        ra[j][2 * e] = v.x;
+        ra[j][2 * e + 1] = v.y;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < TRF; ++i) {
+        const u32x4 v = *reinterpret_cast<const u32x4_any*>(ap[i] + 64 * (int64_t)sg + 8 * j);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) ra[j][4 * i + q] = v[q];
+      }
+    }
+  };
+  auto load_a_guarded = [&](int j, int sg) {                  // zeros past the depth and (rows contiguous) the rows
+    const int64_t k0 = 64 * (int64_t)(seg0 + sg) + 32 * h + 8 * j;
+    if constexpr (ROWS) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        uint32_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int64_t row = r0 + 4 * r + i;
+          v[i] = k0 + e < k && row < m ? A[(k0 + e) * g.sak + row] : 0u;
+        }
+        ra[j][2 * e] = v[0] | (v[1] << 16);
+        ra[j][2 * e + 1] = v[2] | (v[3] << 16);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < TRF; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          uint32_t v[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) v[e] = k0 + 2 * q + e < k ? ap[i][64 * (int64_t)sg + 8 * j + 2 * q + e] : 0u;
+          ra[j][4 * i + q] = v[0] | (v[1] << 16);
+        }
+    }
+  };
+  auto load_b = [&](int j, int sg) {
+    const uint16_t* p = bq + (4 * (int64_t)sg + j) * bstep;
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int n = 0; n < TCF; ++n) rb[j][q][n] = *reinterpret_cast<const u32x4*>(p + (int64_t)q * ncf * 512 + bf[n]);
+  };
+  f32x16 acc[TRF][TCF];
+  float xsq[TRF], xab[TRF];
+#pragma unroll
+  for (int i = 0; i < TRF; ++i) {
+    xsq[i] = xab[i] = 0.f;
+#pragma unroll
+    for (int n = 0; n < TCF; ++n)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][n][e] = 0.f;
+  }
+  auto step = [&](int j) {
+    u32x4 a[TRF];
+    if constexpr (ROWS) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t x0 = ra[j][4 * q], y0 = ra[j][4 * q + 1], x1 = ra[j][4 * q + 2], y1 = ra[j][4 * q + 3];
+        a[0][q] = __builtin_amdgcn_perm(x1, x0, 0x05040100u);             // depths 2 q and 2 q + 1 of row 4 r
+        a[1][q] = __builtin_amdgcn_perm(x1, x0, 0x07060302u);
+        a[2][q] = __builtin_amdgcn_perm(y1, y0, 0x05040100u);
+        a[3][q] = __builtin_amdgcn_perm(y1, y0, 0x07060302u);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < TRF; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[i][q] = ra[j][4 * i + q];
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int n = 0; n < TCF; ++n)
+#pragma unroll
+        for (int i = 0; i < TRF; ++i) acc[i][n] = sdc_pipe::mfma32<DT>(a[i], rb[j][p][n], acc[i][n]);
+    if (do_xn) {
+      constexpr uint32_t ONES = DT == SDC_BF16 ? 0x3F803F80u : 0x3C003C00u;
+#pragma unroll
+      for (int i = 0; i < TRF; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          xsq[i] = pk_dot2<DT>(a[i][q], a[i][q], xsq[i]);
+          xab[i] = pk_dot2<DT>(a[i][q] & 0x7FFF7FFFu, ONES, xab[i]);
+        }
+    }
+  };
+  if (nf > 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      load_a(j, 0);
+      load_b(j, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    for (int sg = 0; sg < nf; ++sg) {
+      const int nx = sg + 1 < nf ? sg + 1 : nf - 1;                        // (past the last: the last again)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        step(j);
+        __builtin_amdgcn_sched_barrier(0);
+        load_a(j, nx);
+        load_b(j, nx);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  if (tail) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      load_a_guarded(j, nf);
+      load_b(j, nf);
+      step(j);
+    }
+  }
+  // fragment row x of fragment i is row 4 x + i of the tile (rows contiguous), or 32 i + x
+  if (do_xn) {
+#pragma unroll
+    for (int i = 0; i < TRF; ++i) {
+      xsq[i] += __shfl_xor(xsq[i], 32, 64);
+      xab[i] += __shfl_xor(xab[i], 32, 64);
+      if (h == 0) {
+        const int row = ROWS ? 4 * r + i : 32 * i + r;
+        xred[w][row][0] = xsq[i];
+        xred[w][row][1] = xab[i];
+      }
+    }
+  }
+  // the waves' sums in LDS, [wave][column][row] (rows padded to RP), then added in wave order
+#pragma unroll
+  for (int n = 0; n < TCF; ++n)
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      float* col = red + (w * TC + 32 * n + r) * RP;
+      if constexpr (ROWS) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          *reinterpret_cast<f32x4*>(col + 4 * (8 * r4 + 4 * h + e)) =
+              f32x4{acc[0][n][4 * r4 + e], acc[1][n][4 * r4 + e], acc[2][n][4 * r4 + e], acc[3][n][4 * r4 + e]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < TRF; ++i)
+          *reinterpret_cast<f32x4*>(col + 32 * i + 8 * r4 + 4 * h) =
+              f32x4{acc[i][n][4 * r4], acc[i][n][4 * r4 + 1], acc[i][n][4 * r4 + 2], acc[i][n][4 * r4 + 3]};
+      }
+    }
+  __syncthreads();
+  if (do_xn && t < TR && r0 + t < m) {
+    float sq = xred[0][t][0], ab = xred[0][t][1];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) {
+      sq += xred[q][t][0];
+      ab += xred[q][t][1];
+    }
+    g.XN[part * 2 * m + r0 + t] = sq;
+    g.XN[part * 2 * m + m + r0 + t] = ab;
+  }
+  float* const Ep = g.E + part * N * m;
+  if (g.et) {
+    // transposed plane [N][m]: an instruction writes two whole columns of the tile, lane l rows 4 (l % 32) .. + 3
+#pragma unroll
+    for (int gq = 0; gq < TC / (2 * NW); ++gq) {
+      const int cl = (w * (TC / (2 * NW)) + gq) * 2 + (lane >> 5);
+      f32x4 v = *reinterpret_cast<const f32x4*>(red + cl * RP + 4 * (lane & 31));
+#pragma unroll
+      for (int q = 1; q < NW; ++q) v += *reinterpret_cast<const f32x4*>(red + (q * TC + cl) * RP + 4 * (lane & 31));
+      const int64_t row = r0 + 4 * (lane & 31), col = c0 + cl;
+      if (col < N) {
+        float* Ec = Ep + col * m;
+        if (row + 4 <= m && m % 4 == 0) {
+          *reinterpret_cast<f32x4*>(Ec + row) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (row + e < m) Ec[row + e] = v[e];
+        }
+      }
+    }
+  } else {
+    // row-major plane [m][N]: an instruction writes 4 rows x 64 columns
+    const int c4 = 4 * (lane & 15);
+#pragma unroll
+    for (int gq = 0; gq < TR / (4 * NW); ++gq) {
+      const int rl = w * (TR / NW) + 4 * gq + (lane >> 4);
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float x = red[(c4 + e) * RP + rl];
+#pragma unroll
+        for (int q = 1; q < NW; ++q) x += red[(q * TC + c4 + e) * RP + rl];
+        v[e] = x;
+      }
+      const int64_t row = r0 + rl, col = c0 + c4;
+      if (row < m) {
+        float* Er = Ep + row * N;
+        if (col + 4 <= N && N % 4 == 0) {
+          *reinterpret_cast<f32x4*>(Er + col) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (col + e < N) Er[col + e] = v[e];
+        }
+      }
+    }
+  }
+}
+
+}  // namespace
+
+// E (and, with g.XN, A's row norms) for one batch of a 16-bit A with unit depth stride, or unit row stride and
+// disjoint depths (g.sak >= g.m >= 4); B in fragment order for the depth rounded up to 64, zeros past it; g.splits
+// (1 .. SDC_MAX_SPLITS) planes.  Returns SDC_EUNSUPPORTED, launching nothing, for other strides.
+int sdc_lane_gemm_launch(int dtype, GemmArgs g, hipStream_t stream) {
+  if (dtype != SDC_BF16 && dtype != SDC_FP16) return SDC_EUNSUPPORTED;
+  const bool rows = g.sak != 1 && g.sam == 1 && g.sak >= g.m && g.m >= 4;
+  if (g.sak != 1 && !rows) return SDC_EUNSUPPORTED;
+  if (g.goffs || g.xf_blocks || g.splits < 1 || g.splits > SDC_MAX_SPLITS || (uintptr_t)g.B % 16 ||
+      (uintptr_t)g.A % 2 || (uintptr_t)g.E % 16 || g.k < 1 || g.k > (1ll << 31))
+    return SDC_EUNSUPPORTED;
+  if (g.m < 1 || g.N < 1) return SDC_EINVAL;
+  const int64_t blocks = g.splits * sdc_cdiv(g.m, TR) * sdc_cdiv(g.N, TC);
+  if (blocks > 0x7FFFFFFF || g.N > 0x7FFFFFFF) return SDC_EUNSUPPORTED;
+  SdcProf prof(g.prof_name ? g.prof_name : "expected_gemm", stream);
+  const dim3 grid((unsigned)blocks), block(64 * NW);
+  if (rows) {
+    if (dtype == SDC_BF16) hipLaunchKernelGGL((lane_gemm_kernel<SDC_BF16, true>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((lane_gemm_kernel<SDC_FP16, true>), grid, block, 0, stream, g);
+  } else {
+    if (dtype == SDC_BF16) hipLaunchKernelGGL((lane_gemm_kernel<SDC_BF16, false>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((lane_gemm_kernel<SDC_FP16, false>), grid, block, 0, stream, g);
+  }
+  SDC_LAUNCH_CHECK();
+  return SDC_OK;
+}

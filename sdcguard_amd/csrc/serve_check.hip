@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256) void serve_pairs_kernel(ScoreArgs a, const flo
 
 // Planes of E and of x's row norms in the workspace: the staged GEMM's, or the tall-tile GEMM's where it has more.
 static int64_t serve_planes(int64_t m, int64_t k, int64_t ncols) {
-  const int64_t s = sdc_expected_splits(m, k, ncols), t = sdc_tall_plan(m, k, ncols).splits;
+  const int64_t s = sdc_expected_splits(m, k, ncols), t = sdc_tall_plan(m, k, ncols, true).splits;
   return s > t ? s : t;
 }
 
@@ -318,7 +318,7 @@ extern "C" int sdc_check_static(int dtype, const void* x, int64_t sxm, int64_t s
   // 23 and 8.7 us, 18944 deep x 56 98 and 16 us; at 4096 rows: 3584 x 56 33 and 18 us, 18944 x 56 123 and
   // 44 us.
   auto expected = [&]() -> int {
-    const TallPlan plan = sdc_tall_plan(m, k, ncols);
+    const TallPlan plan = sdc_tall_plan(m, k, ncols, true);
     if (parts_frag && nparts == 3 && spk == 1 && sxk == 1 && plan.splits > 0) {
       GemmArgs g{};
       g.A = (const uint16_t*)x; g.sam = sxm; g.sak = 1;

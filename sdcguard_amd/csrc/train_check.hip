@@ -15,6 +15,7 @@
 #include "judge.h"
 #include "gemm.h"
 #include "profile.h"
+#include "split.h"
 
 extern "C" int64_t sdc_expected_splits(int64_t m, int64_t k, int64_t ncols);
 
@@ -222,10 +223,9 @@ __device__ __forceinline__ float pow2_ceil(float x) {
   return ldexpf(1.f, f == 0.5f ? e - 1 : e);
 }
 
+// (one wave per block of B)
 template <int DT>
-__global__ __launch_bounds__(64) void b_finish_kernel(BFinishArgs a) {
-  const int lane = threadIdx.x;
-  const int64_t jb = blockIdx.x, bb = blockIdx.y;
+__device__ __forceinline__ void finish_block(const BFinishArgs& a, int64_t jb, int64_t bb, int lane) {
   float st[NSTAT] = {0.f, 0.f, 0.f, 0.f, 0.f};
   for (int64_t kc = lane; kc < a.nkc; kc += 64) {
     const float* p = a.part + ((bb * a.nkc + kc) * a.nb + jb) * NSTAT;
@@ -276,6 +276,66 @@ __global__ __launch_bounds__(64) void b_finish_kernel(BFinishArgs a) {
       a.bias_out[3 * jb + 1] = sg;
       a.bias_out[3 * jb + 2] = mx;
     }
+  }
+}
+
+template <int DT>
+__global__ __launch_bounds__(64) void b_finish_kernel(BFinishArgs a) {
+  finish_block<DT>(a, blockIdx.x, blockIdx.y, threadIdx.x);
+}
+
+// The block sums as three parts in the GEMMs' fragment order, straight from B2^T: 16 bytes of a fragment a thread and
+// part (element e of lane l of fragment (step s, part p, 32 columns f) is column 32 f + l % 32, depth 64 (s / 4) + 32
+// (l / 32) + 8 (s % 4) + e; zero past the columns and the depth).  Consecutive waves take consecutive steps, so a
+// workgroup reads 256 contiguous bytes of each of 32 columns.  Where the parts need no scale (bf16), the first
+// fin_blocks workgroups add up the B side's partial statistics instead (finish_block, a wave each), so one launch
+// does what b_finish, split and the reordering of the parts did in three (12 us each for 64 experts of 2048 x 1408;
+// 4.6 us each at the least).
+struct FragArgs {
+  BFinishArgs fin;
+  int64_t fin_blocks;
+  const float* B2T;                // [batches][ncols][k]
+  const float* scale;              // [batches][ncols] strided by 3 (colstat + 2), or null: 1
+  int64_t ncols, k, ncf, nst, batches;
+  uint16_t* out;                   // a set of nst * 3 * ncf fragments per batch
+};
+
+typedef f32x4 __attribute__((aligned(4))) f32x4_any;
+
+template <int DT>
+__global__ __launch_bounds__(256) void finish_frag_kernel(FragArgs a) {
+  const int t = threadIdx.x, lane = t & 63;
+  if ((int64_t)blockIdx.x < a.fin_blocks) {
+    const int64_t i = (int64_t)blockIdx.x * 4 + (t >> 6);
+    if (i < a.fin.nb * a.batches) finish_block<DT>(a.fin, i % a.fin.nb, i / a.fin.nb, lane);
+    return;
+  }
+  const int64_t set = a.nst * a.ncf, total = a.batches * set;             // (in waves: one step, three fragments)
+  const int64_t stride = ((int64_t)gridDim.x - a.fin_blocks) * 4;
+  for (int64_t i = ((int64_t)blockIdx.x - a.fin_blocks) * 4 + (t >> 6); i < total; i += stride) {
+    const int64_t s = i % a.nst, f = (i / a.nst) % a.ncf, bb = i / set;
+    const int64_t col = 32 * f + lane % 32, kk = 64 * (s / 4) + 32 * (lane / 32) + 8 * (s % 4);
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (col < a.ncols) {
+      const float inv = a.scale ? 1.f / a.scale[(bb * a.ncols + col) * 3] : 1.f;
+      const float* src = a.B2T + (bb * a.ncols + col) * a.k + kk;
+      if (kk + 8 <= a.k) {
+        const f32x4 x = *reinterpret_cast<const f32x4_any*>(src), y = *reinterpret_cast<const f32x4_any*>(src + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = x[e] * inv;
+          v[4 + e] = y[e] * inv;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = kk + e < a.k ? src[e] * inv : 0.f;
+      }
+    }
+    u32x4 pr[3];
+    split8<DT>(v, pr);
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+      *reinterpret_cast<u32x4*>(a.out + (((bb * a.nst + s) * 3 + p) * a.ncf + f) * 512 + 8 * lane) = pr[p];
   }
 }
 
@@ -655,8 +715,9 @@ __global__ __launch_bounds__(256) void grouped_score_kernel(TrainArgs a) {
 struct Layout {
   int64_t nb, rem, ncols, nkc, splits, nbt;
   int64_t kp;                      // depth pitch of the parts (k rounded up to 8: 16-byte aligned columns)
-  int64_t esplits;                 // E and XN planes the workspace holds (the grouped tall GEMM's two at least)
-  int64_t fragb;                   // bytes of one group's parts in fragment order (grouped, depth a multiple of 512)
+  int64_t esplits;                 // E and XN planes the workspace holds (the most any of its GEMMs writes)
+  int64_t fragb;                   // bytes of one group's parts in fragment order (grouped: a depth of whole 512s;
+                                   //   else one batch, its depth rounded up to 64), or 0
   int64_t off_b2t, off_part, off_col, off_bmax, off_bias, off_parts, off_frag, off_e, off_xn, total;
 };
 
@@ -686,9 +747,13 @@ Layout layout(int64_t batch_a, int64_t batch_b, int64_t m, int64_t k, int64_t n,
   L.off_bmax = o; o += al(batch_b * L.nb);
   L.off_bias = o; o += al(3 * L.nb);
   L.off_parts = o; o += al((batch_b * 3 * L.ncols * L.kp + 1) / 2);      // 16-bit parts, two per float
-  L.fragb = grouped && k % TALL_K == 0 ? sdc_parts_fragments_bytes(L.ncols, k) : 0;
+  const int64_t k64 = sdc_cdiv(k, 64) * 64;
+  if (grouped) L.fragb = k % TALL_K == 0 ? sdc_parts_fragments_bytes(L.ncols, k) : 0;
+  else L.fragb = L.nbt == 1 ? sdc_parts_fragments_bytes(L.ncols, k64) : 0;
   L.off_frag = o; o += al(batch_b * L.fragb / 4);
-  L.esplits = L.fragb ? std::max<int64_t>(L.splits, 2) : L.splits;
+  L.esplits = !L.fragb ? L.splits
+                       : std::max<int64_t>(L.splits, grouped ? 2 : std::max(sdc_tall_plan(m, k64, L.ncols, true).splits,
+                                                                            sdc_tall_plan(m, k64, L.ncols, false).splits));
   L.off_e = o; o += al(L.nbt * L.esplits * m * L.ncols);
   L.off_xn = o; o += al(L.nbt * L.esplits * 2 * m);
   L.total = o;
@@ -712,11 +777,13 @@ struct BConsts {
   float* bmaxf;                    // [bB][nb]
   float* bias3;                    // [nb][3]
   uint16_t* parts;                 // [bB][3 * 2nb][kp]
-  uint16_t* frag;                  // the parts in fragment order, [bB][fragb / 2] (grouped), or null
+  uint16_t* frag;                  // the parts in fragment order, [bB][fragb / 2], or null
+  const float* b2t;                // the block sums themselves where `parts` are not made yet (frag is), or null
 };
 
 // The B side: block sums of B and their statistics (b_stage, b_finish), the bias's block sums, and the three parts
-// of the block sums (split).  b2t and part are scratch of layout()'s sizes.
+// of the block sums: in fragment order where bc.frag is set (finish_frag) and k-major otherwise (split); both for a
+// layer's constants (bc.frag set, bc.b2t null).  b2t and part are scratch of layout()'s sizes.
 int stage_b(int dtype, const void* B, int64_t sbb, int64_t sbk, int64_t sbn, int64_t batch_b, int64_t k, int64_t n,
             int64_t bs, const Layout& L, const void* bias, int bias_kind, int64_t sbias_n, const float* s_full,
             const float* s_last, float* b2t, float* part, const BConsts& bc, hipStream_t stream) {
@@ -746,12 +813,28 @@ int stage_b(int dtype, const void* B, int64_t sbb, int64_t sbk, int64_t sbn, int
   fa.colstat = bc.colstat; fa.bmaxf = bc.bmaxf;
   fa.bias = bias_kind == 1 ? (const uint16_t*)bias : nullptr; fa.sbias = sbias_n;
   fa.s_full = s_full; fa.s_last = s_last; fa.bias_out = bc.bias3;
-  {
+  const bool frag_only = bc.frag && bc.b2t;
+  if (!frag_only || dtype != SDC_BF16) {                                 // (fp16: the parts need their scales first)
     SdcProf prof("b_finish", stream);
     dim3 grid((unsigned)L.nb, (unsigned)batch_b);
     if (dtype == SDC_BF16) hipLaunchKernelGGL(b_finish_kernel<SDC_BF16>, grid, dim3(64), 0, stream, fa);
     else hipLaunchKernelGGL(b_finish_kernel<SDC_FP16>, grid, dim3(64), 0, stream, fa);
     SDC_LAUNCH_CHECK();
+  }
+  if (frag_only) {
+    FragArgs ga{};
+    ga.fin = fa;
+    ga.fin_blocks = dtype == SDC_BF16 ? sdc_cdiv(L.nb * batch_b, 4) : 0;
+    ga.B2T = b2t; ga.scale = dtype == SDC_BF16 ? nullptr : bc.colstat + 2;
+    ga.ncols = L.ncols; ga.k = k; ga.ncf = sdc_cdiv(L.ncols, 32); ga.nst = 4 * sdc_cdiv(k, 64); ga.batches = batch_b;
+    ga.out = bc.frag;
+    const int64_t waves = batch_b * ga.nst * ga.ncf;
+    const unsigned grid = (unsigned)(ga.fin_blocks + std::min<int64_t>(sdc_cdiv(waves, 4), 4096));
+    SdcProf prof("finish_frag", stream);
+    if (dtype == SDC_BF16) hipLaunchKernelGGL(finish_frag_kernel<SDC_BF16>, dim3(grid), dim3(256), 0, stream, ga);
+    else hipLaunchKernelGGL(finish_frag_kernel<SDC_FP16>, dim3(grid), dim3(256), 0, stream, ga);
+    SDC_LAUNCH_CHECK();
+    return SDC_OK;
   }
   // the three parts of B2 / scale (scale: every third float of colstat, stride 3 per column)
   int rc = sdc_split_launch(dtype, b2t, bc.colstat + 2, L.ncols * 3, 3, L.ncols, k, L.kp, batch_b, bc.parts, stream);
@@ -781,8 +864,13 @@ int run_check(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, i
   float* ws = (float*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
   const float* s_full = sign_table + (bs - 1) * 128;
   const float* s_last = L.rem ? sign_table + (L.rem - 1) * 128 : s_full;
+  // the parts go straight to fragment order where a GEMM that reads it takes A: one batch of a 16-bit A with unit
+  // depth stride or unit row stride, or grouped rows 16-byte aligned (check_with makes the k-major parts after all
+  // where every such GEMM refuses)
+  const bool rows16 = sak == 1 && sam % 8 == 0 && (uintptr_t)A % 16 == 0;
+  const bool frag = L.fragb && (grouped ? rows16 && batch_b <= 1024 : (sak == 1 || (sam == 1 && sak >= m && m >= 4)));
   const BConsts bc{ws + L.off_col, ws + L.off_bmax, ws + L.off_bias, (uint16_t*)(ws + L.off_parts),
-                   L.fragb ? (uint16_t*)(ws + L.off_frag) : nullptr};
+                   frag ? (uint16_t*)(ws + L.off_frag) : nullptr, frag ? ws + L.off_b2t : nullptr};
   int rc = stage_b(dtype, B, sbb, sbk, sbn, batch_b, k, n, bs, L, bias, bias_kind, sbias_n, s_full, s_last,
                    ws + L.off_b2t, ws + L.off_part, bc, stream);
   if (rc != SDC_OK) return rc;
@@ -812,6 +900,22 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
   int rc = SDC_EUNSUPPORTED;
   int64_t splits = L.splits;
   bool e_t = c_t;
+  if (!grouped && bc.frag) {
+    // the tall-tile GEMM where A's rows allow whole lines, else the one that reads A of any alignment and either
+    // unit stride
+    const int64_t k64 = sdc_cdiv(k, 64) * 64;
+    GemmArgs gt = g;
+    gt.B = bc.frag; gt.sbb = 0; gt.sbc = 0;
+    TallPlan plan = sdc_tall_plan(m, k64, L.ncols, true);
+    gt.splits = plan.splits; gt.short_rows = plan.short_rows;
+    rc = sdc_rs_gemm_tall_launch(dtype, gt, 0, stream);
+    if (rc == SDC_EUNSUPPORTED) {
+      gt.splits = sdc_tall_plan(m, k64, L.ncols, false).splits;
+      gt.short_rows = 0;
+      rc = sdc_lane_gemm_launch(dtype, gt, stream);
+    }
+    if (rc == SDC_OK) splits = gt.splits;
+  }
   if (grouped && bc.frag) {
     // the tall-tile GEMM over SDC_GROUPED_TALL_SPLITS depth parts: E transposed, the groups' fragments L.fragb bytes
     // apart
@@ -824,7 +928,13 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
       e_t = true;
     }
   }
-  if (rc == SDC_EUNSUPPORTED) rc = sdc_gemm_launch(dtype, g, nbt, stream);
+  if (rc == SDC_EUNSUPPORTED) {
+    if (bc.b2t) {
+      rc = sdc_split_launch(dtype, bc.b2t, bc.colstat + 2, L.ncols * 3, 3, L.ncols, k, L.kp, batch_b, bc.parts, stream);
+      if (rc != SDC_OK) return rc;
+    }
+    rc = sdc_gemm_launch(dtype, g, nbt, stream);
+  }
   if (rc != SDC_OK) return rc;
 
   TrainArgs ta{};
@@ -931,7 +1041,8 @@ ConstsLayout consts_layout(int64_t groups, int64_t k, int64_t n, int64_t bs) {
 BConsts consts_at(void* consts, const ConstsLayout& c) {
   uint8_t* p = (uint8_t*)consts;
   return BConsts{(float*)(p + c.off_col), (float*)(p + c.off_bmax), (float*)(p + c.off_bias),
-                 (uint16_t*)(p + c.off_parts), c.total > c.off_frag ? (uint16_t*)(p + c.off_frag) : nullptr};
+                 (uint16_t*)(p + c.off_parts), c.total > c.off_frag ? (uint16_t*)(p + c.off_frag) : nullptr,
+                 nullptr};
 }
 }  // namespace
 

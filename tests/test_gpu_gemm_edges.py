@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from oracle import serve_check
+from oracle import abft, serve_check
 from tests.test_gpu_serve import run_gpu
 from tests.test_oracle_golden import gemm_slack, z_close
 
@@ -28,3 +28,40 @@ def test_serving_rows_and_depths(m, k, n, dt):
     ok = z_close(zs.reshape(-1), o.z.reshape(-1), gemm_slack(o.csb, o.den).reshape(-1))
     assert ok.all(), (np.nonzero(~ok)[0][:5], zs.reshape(-1)[~ok][:5], o.z.reshape(-1)[~ok][:5])
     assert st[0, 2] == 1 and st[0, 3] == 0
+
+
+def _operand(rows, cols, layout, g, t, std):
+    """(rows, cols) of dtype t in a layout: row- or column-contiguous, at an odd offset of odd-strided storage, or with
+    neither stride one."""
+    if layout == "rows":
+        return (torch.randn(rows, cols, generator=g) * std).to(t).cuda()
+    if layout == "cols":
+        return (torch.randn(cols, rows, generator=g) * std).to(t).cuda().t()
+    if layout == "odd":
+        return (torch.randn(rows, cols + 5, generator=g) * std).to(t).cuda()[:, 3:3 + cols]
+    if layout == "cols_odd":
+        return (torch.randn(cols, rows + 5, generator=g) * std).to(t).cuda()[:, 3:3 + rows].t()
+    if layout == "expanded":
+        return (torch.randn(1, cols, generator=g) * std).to(t).cuda().expand(rows, cols)
+    return (torch.randn(rows, 2 * cols, generator=g) * std).to(t).cuda()[:, ::2]
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("la", ["rows", "cols", "odd", "cols_odd", "expanded", "strided"])
+@pytest.mark.parametrize("m,k,n,lb", [(1, 1, 1, "rows"), (3, 64, 130, "cols"), (37, 63, 128, "rows"),
+                                      (128, 128, 256, "cols"), (131, 65, 300, "odd"), (257, 1030, 513, "cols_odd"),
+                                      (514, 320, 4300, "rows")])
+def test_training_operand_layouts(m, k, n, lb, la, dt):
+    """Every layout of A through the GEMM its strides and depth pick, every checksum's score against the oracle's."""
+    from sdcguard_amd import matmul_zscores
+    g = torch.Generator().manual_seed(m + k + n)
+    t = torch.bfloat16 if dt == "bf16" else torch.float16
+    A, B = _operand(m, k, la, g, t, 1.0), _operand(k, n, lb, g, t, 0.1)
+    C = (A.float().cpu() @ B.float().cpu()).to(t)
+    scores = torch.full((1, m, -(-n // 128), 2), -7.0, device="cuda")
+    row = matmul_zscores(A, B, C.cuda(), scores_out=scores).result.tolist()
+    o = abft.zscores(A.float().cpu().numpy(), B.float().cpu().numpy(), C.float().numpy(), dtype=dt, seed=1)
+    z = scores.cpu().numpy().reshape(-1)
+    ok = z_close(z, o.z.reshape(-1), gemm_slack(o.csb, o.den).reshape(-1))
+    assert ok.all(), (np.nonzero(~ok)[0][:5], z[~ok][:5], o.z.reshape(-1)[~ok][:5])
+    assert row[2] == 0
