@@ -14,10 +14,13 @@ struct YView {
   const uint16_t* y;
   int64_t sb, sm, sn;
   int64_t m, nb, bs, rem, npairs;      // npairs = batches * m * nb (flat pair index p = (b * m + r) * nb + jb)
-  int vec;                             // 16-byte loads allowed (sn == 1, aligned rows, bs % 8 == 0)
+  int vec;                             // 16-byte loads (sn == 1; any alignment)
   const float* s_full;                 // +-1 pattern of width bs (a 128-entry row of the sign table)
   const float* s_last;                 // +-1 pattern of width rem
 };
+
+// Whether any block is narrower than 128 in a row read in 16-byte pieces
+static inline bool blocks_narrow(const YView& v) { return v.vec && (v.rem != 0 || v.bs != 128); }
 
 __device__ __forceinline__ void pair_index(const YView& v, int64_t p, int64_t& b, int64_t& r, int64_t& jb) {
   const uint32_t rr = (uint32_t)p / (uint32_t)v.nb;
@@ -67,30 +70,81 @@ __device__ __forceinline__ void acc8(u32x4 v, const uint32_t* sg2, float& pl, fl
   }
 }
 
+// 16 bytes at any 2-byte address (global loads take any), read once
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+__device__ __forceinline__ u32x4 load16_any(const uint16_t* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
+}
+
+// v's elements moved down by sh (0 .. 8), zeros from the top
+__device__ __forceinline__ u32x4 drop_low(u32x4 v, int sh) {
+  if (sh & 1) {
+    v.x = __builtin_amdgcn_alignbit(v.y, v.x, 16);
+    v.y = __builtin_amdgcn_alignbit(v.z, v.y, 16);
+    v.z = __builtin_amdgcn_alignbit(v.w, v.z, 16);
+    v.w = v.w >> 16;
+  }
+  if (sh & 2) v = u32x4{v.y, v.z, v.w, 0u};
+  if (sh & 4) v = u32x4{v.z, v.w, 0u, 0u};
+  if (sh & 8) v = u32x4{0u, 0u, 0u, 0u};
+  return v;
+}
+
+// The 8 elements at columns c0 .. c0 + 7 of a block of `wid` columns (row: the block's first), zeros past wid: the 16
+// bytes are read from the block's last 8 columns back where c0 + 8 passes its end, so nothing past the row is read;
+// the block's end must be at least 8 columns from its row's start.
+__device__ __forceinline__ u32x4 load8_upto(const uint16_t* row, int c0, int wid) {
+  const int off = c0 + 8 <= wid ? c0 : wid - 8, sh = c0 - off;
+  const u32x4 v = load16_any(row + off);
+  return sh > 0 ? drop_low(v, sh < 8 ? sh : 8) : v;
+}
+
+// The signs of 8 columns of a pattern (a table row: zeros past its width) as packed pairs
+template <int DT>
+__device__ __forceinline__ void pack_signs8(const float* sp, uint32_t* sg2) {
+  constexpr uint32_t POS = DT == SDC_BF16 ? 0x3F80u : 0x3C00u, NEG = DT == SDC_BF16 ? 0xBF80u : 0xBC00u;
+  const f32x4 s0 = *reinterpret_cast<const f32x4*>(sp), s1 = *reinterpret_cast<const f32x4*>(sp + 4);
+  sg2[0] = (s0.x < 0.f ? NEG : POS) | ((s0.y < 0.f ? NEG : POS) << 16);
+  sg2[1] = (s0.z < 0.f ? NEG : POS) | ((s0.w < 0.f ? NEG : POS) << 16);
+  sg2[2] = (s1.x < 0.f ? NEG : POS) | ((s1.y < 0.f ? NEG : POS) << 16);
+  sg2[3] = (s1.z < 0.f ? NEG : POS) | ((s1.w < 0.f ? NEG : POS) << 16);
+}
+
 // The four sums of the (row, block) pair each lane keeps: a wave reads 64 consecutive pairs starting at `base`;
 // lane l ends up with pair base + (l & 3) * 16 + (l >> 2).  Four lanes share a pair in each of four rounds; all
-// sixteen 16-byte loads are issued before any is used (256 bytes per lane in flight).  Pairs that are not full
-// 128-wide vector-loadable blocks (a narrower last block, strided y) take an element-wise path.
-template <int DT>
+// sixteen 16-byte loads are issued before any is used (256 bytes per lane in flight).  A block narrower than 128 (a
+// row's last) is read the same way, its columns past the end dropped, with its own width's signs: 577-wide rows, a
+// fifth of whose blocks are 65 wide, take 41 us for 64 MB, from 114 us with element loads for every block of
+// rows that are not 16-byte aligned.  Strided rows, and rows of fewer than 8 columns, take an element-wise path.
+// NARROW: whether narrower blocks are read so (they cost 20 registers, a wave a SIMD: 4096 x 14336 35 and 42 us
+// without and with them, so passes over whole blocks leave them out; blocks_narrow).
+template <int DT, bool NARROW>
 __device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane, const uint32_t* sg2, float& my_pl,
                                           float& my_sg, float& my_sq, float& my_ab) {
   const int q = lane & 3;
-  bool full[4];
+  int how[4];                           // 0: elements, 1: a full block, 2: a narrower one
   u32x4 v[4][4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const int64_t p = base + g * 16 + (lane >> 2);
-    full[g] = false;
+    how[g] = 0;
     if (p < a.npairs && a.vec) {
       int64_t b, r, jb;
       pair_index(a, p, b, r, jb);
       const bool last = (jb == a.nb - 1) && (a.rem > 0);
-      if (!last && a.bs == 128) {
-        full[g] = true;
-        const uint16_t* yr = a.y + b * a.sb + r * a.sm + jb * 128;
+      const int wid = (int)(last ? a.rem : a.bs);
+      const uint16_t* yr = a.y + b * a.sb + r * a.sm + jb * a.bs;
+      if (wid == 128) {
+        how[g] = 1;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          v[g][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(yr + 8 * (q + 4 * j)));
+        for (int j = 0; j < 4; ++j) v[g][j] = load16_any(yr + 8 * (q + 4 * j));
+      } else if (NARROW && jb * a.bs + wid >= 8) {
+        how[g] = 2;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int c0 = 8 * (q + 4 * j);
+          v[g][j] = load16_any(yr + (c0 + 8 <= wid ? c0 : wid - 8));
+        }
       }
     }
   }
@@ -99,29 +153,39 @@ __device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane
   for (int g = 0; g < 4; ++g) {
     const int64_t p = base + g * 16 + (lane >> 2);
     float pl = 0.f, sg = 0.f, sq = 0.f, ab = 0.f;
-    if (full[g]) {
+    if (how[g] == 1) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc8<DT>(v[g][j], &sg2[j * 4], pl, sg, sq, ab);
     } else if (p < a.npairs) {
       int64_t b, r, jb;
       pair_index(a, p, b, r, jb);
       const bool last = (jb == a.nb - 1) && (a.rem > 0);
-      const int64_t wid = last ? a.rem : a.bs;
-      const uint16_t* yr = a.y + b * a.sb + r * a.sm + jb * a.bs * a.sn;
+      const int wid = (int)(last ? a.rem : a.bs);
       const float* sp = last ? a.s_last : a.s_full;
-#pragma unroll 1
-      for (int j = 0; j < 4; ++j)
-#pragma unroll 1
-        for (int e = 0; e < 8; ++e) {
-          const int c = 8 * (q + 4 * j) + e;
-          if (c < wid) {
-            float x = half_to_f32<DT>(yr[c * a.sn]);
-            pl += x;
-            sg = fmaf(x, sp[c], sg);
-            sq = fmaf(x, x, sq);
-            ab += fabsf(x);
-          }
+      if (NARROW && how[g] == 2) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int c0 = 8 * (q + 4 * j), sh = c0 + 8 - wid;
+          uint32_t ns[4];
+          pack_signs8<DT>(sp + c0, ns);
+          acc8<DT>(sh > 0 ? drop_low(v[g][j], sh < 8 ? sh : 8) : v[g][j], ns, pl, sg, sq, ab);
         }
+      } else {
+        const uint16_t* yr = a.y + b * a.sb + r * a.sm + jb * a.bs * a.sn;
+#pragma unroll 1
+        for (int j = 0; j < 4; ++j)
+#pragma unroll 1
+          for (int e = 0; e < 8; ++e) {
+            const int c = 8 * (q + 4 * j) + e;
+            if (c < wid) {
+              float x = half_to_f32<DT>(yr[c * a.sn]);
+              pl += x;
+              sg = fmaf(x, sp[c], sg);
+              sq = fmaf(x, x, sq);
+              ab += fabsf(x);
+            }
+          }
+      }
     }
     pl = quad_sum(pl); sg = quad_sum(sg); sq = quad_sum(sq); ab = quad_sum(ab);
     if (q == g) { my_pl = pl; my_sg = sg; my_sq = sq; my_ab = ab; }
@@ -132,15 +196,6 @@ __device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane
 // table row holds 128 entries (zeros past its width), so these loads need no bounds test.
 template <int DT>
 __device__ __forceinline__ void lane_signs(const YView& a, int q, uint32_t* sg2) {
-  constexpr uint32_t POS = DT == SDC_BF16 ? 0x3F80u : 0x3C00u, NEG = DT == SDC_BF16 ? 0xBF80u : 0xBC00u;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const f32x4 s0 = *reinterpret_cast<const f32x4*>(a.s_full + 8 * (q + 4 * j));
-    const f32x4 s1 = *reinterpret_cast<const f32x4*>(a.s_full + 8 * (q + 4 * j) + 4);
-    sg2[j * 4 + 0] = (s0.x < 0.f ? NEG : POS) | ((s0.y < 0.f ? NEG : POS) << 16);
-    sg2[j * 4 + 1] = (s0.z < 0.f ? NEG : POS) | ((s0.w < 0.f ? NEG : POS) << 16);
-    sg2[j * 4 + 2] = (s1.x < 0.f ? NEG : POS) | ((s1.y < 0.f ? NEG : POS) << 16);
-    sg2[j * 4 + 3] = (s1.z < 0.f ? NEG : POS) | ((s1.w < 0.f ? NEG : POS) << 16);
-  }
+  for (int j = 0; j < 4; ++j) pack_signs8<DT>(a.s_full + 8 * (q + 4 * j), &sg2[j * 4]);
 }
-

@@ -1232,8 +1232,8 @@ int sdc_rs_gemm_launch(int dtype, GemmArgs g, int role, hipStream_t stream) {
 
 // Row tiles (32, 64 or 128 rows) and depth parts of the tall-tile GEMM for 16-bit rows, m x k against N columns: the
 // shortest tile that holds a short m whole (16 rows against 128-row tiles multiply seven eighths padding), then the
-// number of parts, at most SDC_MAX_SPLITS, with the least rounds of 256 workgroups x (set-up + a wave's segments) +
-// the planes' traffic.  The set-up (about 6 us: the first loads and the epilogue), a segment's time (1.6 us for 128
+// number of parts, at most SDC_MAX_GEMM_SPLITS, with the least rounds of 256 workgroups x (set-up + a wave's segments) +
+// the planes' traffic and, past the SDC_MAX_SPLITS that a scoring pass loads at once, their latency.  The set-up (about 6 us: the first loads and the epilogue), a segment's time (1.6 us for 128
 // rows, 0.7 us for 32) and 5 TB/s for a plane written and read back are this GEMM's as measured on MI355X.
 TallPlan sdc_tall_plan(int64_t m, int64_t k, int64_t N, bool short_ok) {
   TallPlan p{0, 0};
@@ -1243,8 +1243,9 @@ TallPlan sdc_tall_plan(int64_t m, int64_t k, int64_t N, bool short_ok) {
   const int64_t tiles = sdc_cdiv(m, tr) * sdc_cdiv(N, 64);
   const double seg = 0.4 + 1.2 * (double)tr / 128.0, plane = 8e-6 * (double)m * (double)N / 5.0;
   double best = 0.0;
-  for (int64_t s = 1; s <= SDC_MAX_SPLITS && s * nw <= nseg + nw - 1; ++s) {
-    const double c = (double)sdc_cdiv(tiles * s, 256) * (6.0 + seg * (double)sdc_cdiv(nseg, nw * s)) + plane * (double)s;
+  for (int64_t s = 1; s <= SDC_MAX_GEMM_SPLITS && s * nw <= nseg + nw - 1; ++s) {
+    const double c = (double)sdc_cdiv(tiles * s, 256) * (6.0 + seg * (double)sdc_cdiv(nseg, nw * s)) +
+                     plane * (double)s + (s > SDC_MAX_SPLITS ? 0.2 * (double)(s - SDC_MAX_SPLITS) : 0.0);
     if (p.splits == 0 || c < best) {
       p.splits = s;
       best = c;
@@ -1254,7 +1255,7 @@ TallPlan sdc_tall_plan(int64_t m, int64_t k, int64_t N, bool short_ok) {
 }
 
 // The tall-tile variant: 128 x 64 tiles (g.short_rows 1 or 2: 64 x 64 or 32 x 64; for a 16-bit A only with g.XN and
-// no groups) over g.splits (1 .. SDC_MAX_SPLITS) depth parts, one plane of E per part (the depth a multiple of 64, of
+// no groups) over g.splits (1 .. SDC_MAX_GEMM_SPLITS) depth parts, one plane of E per part (the depth a multiple of 64, of
 // 128 for a byte A, dealt to the parts' waves in whole segments; A's rows 16-byte aligned); with g.XN set, also A's
 // row norms, one plane per part.  dtype SDC_FP8: an fp8 e4m3 A widened to bf16 (B's parts bf16).  With g.goffs
 // (16-bit A only): rows grouped by the groups' cumulative ends, group q's fragments at g.B + q g.sbb, row norms
@@ -1263,7 +1264,7 @@ int sdc_rs_gemm_tall_launch(int dtype, GemmArgs g, int role, hipStream_t stream)
   if (dtype != SDC_BF16 && dtype != SDC_FP16 && dtype != SDC_FP8 && dtype != SDC_I8) return SDC_EUNSUPPORTED;
   const bool byte_a = dtype == SDC_FP8 || dtype == SDC_I8;
   const int64_t es = byte_a ? 1 : 2, kmul = byte_a ? 128 : 64;
-  if (g.splits < 1 || g.splits > SDC_MAX_SPLITS || g.sak != 1 || g.k < kmul || g.k % kmul ||
+  if (g.splits < 1 || g.splits > SDC_MAX_GEMM_SPLITS || g.sak != 1 || g.k < kmul || g.k % kmul ||
       g.k / kmul > 0xFFFFFF || (g.sam * es) % 16 ||
       ((uintptr_t)g.A | (uintptr_t)g.B) % 16 || (!g.et && (g.goffs || ((uintptr_t)g.E % 16))))
     return SDC_EUNSUPPORTED;

@@ -25,7 +25,7 @@ namespace {
 constexpr int NW = 4, TRF = 4, TCF = 2, TR = 128, TC = 64, RP = TR + 4;
 
 typedef u32x2 __attribute__((aligned(2))) u32x2_any;        // 8 and 16 bytes at any 2-byte address
-typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+typedef u32x4 __attribute__((aligned(2))) u32x4_lane;
 
 // ROWS: rows contiguous (g.sam 1, g.sak >= g.m >= 4); else depth contiguous (g.sak 1)
 template <int DT, bool ROWS>
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(64 * NW, 1) void lane_gemm_kernel(GemmArgs g) {
     } else {
 #pragma unroll
       for (int i = 0; i < TRF; ++i) {
-        const u32x4 v = *reinterpret_cast<const u32x4_any*>(ap[i] + 64 * (int64_t)sg + 8 * j);
+        const u32x4 v = *reinterpret_cast<const u32x4_lane*>(ap[i] + 64 * (int64_t)sg + 8 * j);
 #pragma unroll
         for (int q = 0; q < 4; ++q) ra[j][4 * i + q] = v[q];
       }
@@ -294,12 +294,12 @@ __global__ __launch_bounds__(64 * NW, 1) void lane_gemm_kernel(GemmArgs g) {
 
 // E (and, with g.XN, A's row norms) for one batch of a 16-bit A with unit depth stride, or unit row stride and
 // disjoint depths (g.sak >= g.m >= 4); B in fragment order for the depth rounded up to 64, zeros past it; g.splits
-// (1 .. SDC_MAX_SPLITS) planes.  Returns SDC_EUNSUPPORTED, launching nothing, for other strides.
+// (1 .. SDC_MAX_GEMM_SPLITS) planes.  Returns SDC_EUNSUPPORTED, launching nothing, for other strides.
 int sdc_lane_gemm_launch(int dtype, GemmArgs g, hipStream_t stream) {
   if (dtype != SDC_BF16 && dtype != SDC_FP16) return SDC_EUNSUPPORTED;
   const bool rows = g.sak != 1 && g.sam == 1 && g.sak >= g.m && g.m >= 4;
   if (g.sak != 1 && !rows) return SDC_EUNSUPPORTED;
-  if (g.goffs || g.xf_blocks || g.splits < 1 || g.splits > SDC_MAX_SPLITS || (uintptr_t)g.B % 16 ||
+  if (g.goffs || g.xf_blocks || g.splits < 1 || g.splits > SDC_MAX_GEMM_SPLITS || (uintptr_t)g.B % 16 ||
       (uintptr_t)g.A % 2 || (uintptr_t)g.E % 16 || g.k < 1 || g.k > (1ll << 31))
     return SDC_EUNSUPPORTED;
   if (g.m < 1 || g.N < 1) return SDC_EINVAL;

@@ -9,6 +9,8 @@
 //      of squares, of |values|) and add them up with two DPP steps; over four rounds each lane keeps one pair's
 //      sums, then scores it with the reference's noise model.  The workgroup's worst key goes into the layer's
 //      state row with one integer atomic maximum (only when it raises the row), counts with atomic adds.
+#include <type_traits>
+
 #include "blocksums.h"
 #include "judge.h"
 #include "gemm.h"
@@ -47,9 +49,10 @@ struct LaneBest {
   int unk = 0;
 };
 
-// Pair p's expected sums and x row norms over the GEMM's NS depth-split planes (NS at most SDC_MAX_SPLITS), all
+// Pair p's expected sums and x row norms over the GEMM's first NS depth-split planes (NS at most SDC_MAX_SPLITS), all
 // loads issued before any is used and unconditional: a split index past a.splits reads split 0 (added nowhere), a
-// pair past the last reads the last pair's (scored nowhere).
+// pair past the last reads the last pair's (scored nowhere).  Planes past NS are added in order when it is scored
+// (MORE).
 template <int NS>
 struct PairE {
   float2 ev[NS];
@@ -75,7 +78,7 @@ __device__ __forceinline__ PairE<NS> load_pair_e(const ScoreArgs& a, int64_t p) 
 }
 
 // Scores pair p (skipped when p >= npairs) from its four sums and its loaded planes into the lane's running worst.
-template <int DT, int NS>
+template <int DT, int NS, bool MORE>
 __device__ __forceinline__ void score_pair_e(const ScoreArgs& a, int64_t p, float pl, float sg, float sq, float ab,
                                              const PairE<NS>& pe, LaneBest& best) {
   if (p >= a.npairs) return;
@@ -91,6 +94,18 @@ __device__ __forceinline__ void score_pair_e(const ScoreArgs& a, int64_t p, floa
       e1 += pe.ev[s].y;
       asq += pe.xa[s];
       asum += pe.xb[s];
+    }
+  }
+  if (MORE && a.splits > NS) {
+    const float* ep = a.E + r * a.ncols + 2 * jb;
+    const float* xp = a.XN + r;
+#pragma unroll 8
+    for (int64_t s = NS; s < a.splits; ++s) {
+      const float2 v = *reinterpret_cast<const float2*>(ep + s * a.m * a.ncols);
+      e0 += v.x;
+      e1 += v.y;
+      asq += xp[s * 2 * a.m];
+      asum += xp[s * 2 * a.m + a.m];
     }
   }
   PairScore ps;
@@ -125,7 +140,7 @@ template <int DT>
 __device__ __forceinline__ void score_pair(const ScoreArgs& a, int64_t p, float pl, float sg, float sq, float ab,
                                            LaneBest& best) {
   if (p >= a.npairs) return;
-  score_pair_e<DT, SDC_MAX_SPLITS>(a, p, pl, sg, sq, ab, load_pair_e<SDC_MAX_SPLITS>(a, p), best);
+  score_pair_e<DT, SDC_MAX_SPLITS, true>(a, p, pl, sg, sq, ab, load_pair_e<SDC_MAX_SPLITS>(a, p), best);
 }
 
 // The workgroup's worst key into the layer's state row (one atomic maximum, only when it raises the row), the
@@ -193,7 +208,8 @@ __device__ __forceinline__ void report_wg(const ScoreArgs& a, LaneBest best) {
 // v1 (one launch after the GEMM): sums and scores in the same pass over y.  Each wave walks tiles of 64 pairs
 // with a grid stride and keeps its worst key; the workgroup reports once at the end.  A tile's expected sums (NS
 // planes: 2 from the tall-tile GEMM) are loaded before its outputs, so both arrive in one round trip.
-template <int DT, int NS>
+// GEN: y has blocks narrower than 128, or the GEMM more than NS planes.
+template <int DT, int NS, bool GEN>
 __global__ __launch_bounds__(256) void serve_fused_kernel(ScoreArgs a) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, q = lane & 3;
   uint32_t sg2[16];
@@ -204,8 +220,8 @@ __global__ __launch_bounds__(256) void serve_fused_kernel(ScoreArgs a) {
     const int64_t base = tile * 64, p = base + q * 16 + (lane >> 2);
     const PairE<NS> pe = load_pair_e<NS>(a, p);
     float pl, sg, sq, ab;
-    pair_sums<DT>(a.yv, base, lane, sg2, pl, sg, sq, ab);
-    score_pair_e<DT, NS>(a, p, pl, sg, sq, ab, pe, best);
+    pair_sums<DT, GEN>(a.yv, base, lane, sg2, pl, sg, sq, ab);
+    score_pair_e<DT, NS, GEN>(a, p, pl, sg, sq, ab, pe, best);
   }
   report_wg<DT>(a, best);
 }
@@ -221,7 +237,7 @@ __global__ __launch_bounds__(256) void serve_sums_kernel(ScoreArgs a, float* __r
   for (int64_t tile = (int64_t)blockIdx.x * 4 + w; tile < tiles; tile += (int64_t)gridDim.x * 4) {
     const int64_t base = tile * 64;
     float pl, sg, sq, ab;
-    pair_sums<DT>(a.yv, base, lane, sg2, pl, sg, sq, ab);
+    pair_sums<DT, true>(a.yv, base, lane, sg2, pl, sg, sq, ab);
     const int64_t p = base + q * 16 + (lane >> 2);
     if (p < a.npairs) {
       sums[p] = pl;
@@ -308,7 +324,7 @@ extern "C" int sdc_check_static(int dtype, const void* x, int64_t sxm, int64_t s
   a.zdump = scores_out;
   a.packed = (const f32x4*)block_consts;
   if (block_consts && ((uintptr_t)block_consts % 16)) return SDC_EINVAL;
-  a.vec = (syn == 1) && (sym % 8 == 0) && (bs % 8 == 0) && ((uintptr_t)y % 16 == 0);
+  a.vec = syn == 1;
   a.yv.vec = a.vec;
   if (cap_meta && (!cap_data || cap_w < bs)) return SDC_EINVAL;
   // The expected side: the register-streamed tall-tile GEMM (row-major planes, x's row norms in the same pass) where
@@ -340,15 +356,19 @@ extern "C" int sdc_check_static(int dtype, const void* x, int64_t sxm, int64_t s
     int rc = expected();
     if (rc != SDC_OK) return rc;
     SdcProf prof("serve_fused", stream);
-    constexpr int MS = SDC_MAX_SPLITS;
-    if (dtype == SDC_BF16 && a.splits <= 2)
-      hipLaunchKernelGGL((serve_fused_kernel<SDC_BF16, 2>), dim3(grid), dim3(256), 0, stream, a);
-    else if (dtype == SDC_BF16)
-      hipLaunchKernelGGL((serve_fused_kernel<SDC_BF16, MS>), dim3(grid), dim3(256), 0, stream, a);
-    else if (a.splits <= 2)
-      hipLaunchKernelGGL((serve_fused_kernel<SDC_FP16, 2>), dim3(grid), dim3(256), 0, stream, a);
-    else
-      hipLaunchKernelGGL((serve_fused_kernel<SDC_FP16, MS>), dim3(grid), dim3(256), 0, stream, a);
+    auto go = [&](auto dt, auto ns, auto gen) {
+      hipLaunchKernelGGL((serve_fused_kernel<decltype(dt)::value, decltype(ns)::value, decltype(gen)::value>),
+                         dim3(grid), dim3(256), 0, stream, a);
+    };
+    auto with_dt = [&](auto dt) {
+      const bool narrow = blocks_narrow(a.yv);
+      if (a.splits <= 2 && !narrow) go(dt, std::integral_constant<int, 2>{}, std::false_type{});
+      else if (a.splits <= SDC_MAX_SPLITS && !narrow)
+        go(dt, std::integral_constant<int, SDC_MAX_SPLITS>{}, std::false_type{});
+      else go(dt, std::integral_constant<int, SDC_MAX_SPLITS>{}, std::true_type{});
+    };
+    if (dtype == SDC_BF16) with_dt(std::integral_constant<int, SDC_BF16>{});
+    else with_dt(std::integral_constant<int, SDC_FP16>{});
     SDC_LAUNCH_CHECK();
     return SDC_OK;
   }

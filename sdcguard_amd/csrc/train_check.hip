@@ -11,6 +11,8 @@
 //   3. split + expected_gemm (expected_gemm.hip): B2 as three parts, E = A @ B2 on MFMA, plus A's row norms;
 //   4. train_score: one persistent pass over C scoring every (batch, row, block) pair, worst key and unjudged count
 //      into the check's result row with atomics.
+#include <type_traits>
+
 #include "blocksums.h"
 #include "judge.h"
 #include "gemm.h"
@@ -37,7 +39,8 @@ struct BStageArgs {
 
 __device__ __forceinline__ float nan_inf(float v) { return v == v ? fabsf(v) : __builtin_inff(); }
 
-template <int DT>
+// NARROW: B has blocks narrower than 128
+template <int DT, bool NARROW>
 __global__ __launch_bounds__(256) void b_stage_kernel(BStageArgs a) {
   __shared__ float red[4][NSTAT];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, q = t & 3;
@@ -49,11 +52,16 @@ __global__ __launch_bounds__(256) void b_stage_kernel(BStageArgs a) {
   float pl = 0.f, sg = 0.f, mx = 0.f;
   if (kk < a.k) {
     const uint16_t* row = a.B + bb * a.sbb + kk * a.sbk + jb * a.bs * a.sbn;
-    if (a.vec && wid == 128) {
+    if (a.vec && (NARROW ? jb * a.bs + wid >= 8 : wid == 128)) {
+      u32x4 vv[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        vv[j] = NARROW ? load8_upto(row, 8 * (q + 4 * j), (int)wid)
+                       : *reinterpret_cast<const u32x4_any*>(row + 8 * (q + 4 * j));
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int c0 = 8 * (q + 4 * j);
-        const u32x4 v = *reinterpret_cast<const u32x4*>(row + c0);
+        const u32x4 v = vv[j];
         const f32x4 s0 = *reinterpret_cast<const f32x4*>(sp + c0);
         const f32x4 s1 = *reinterpret_cast<const f32x4*>(sp + c0 + 4);
         const float x[8] = {lo_of<DT>(v.x), hi_of<DT>(v.x), lo_of<DT>(v.y), hi_of<DT>(v.y),
@@ -146,13 +154,13 @@ __global__ __launch_bounds__(256) void b_stage_t_kernel(BStageArgs a) {
     u32x4 v[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      v[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(base + (cg + 8 * i) * a.sbn));
+      v[i] = load16_any(base + (cg + 8 * i) * a.sbn);
 #pragma unroll
     for (int i = 0; i < 16; ++i) add8(v[i], sp[cg + 8 * i]);
   } else if (a.vec && kk0 + 8 <= a.k) {
 #pragma unroll 4
     for (int c = cg; c < wid; c += 8)
-      add8(__builtin_nontemporal_load(reinterpret_cast<const u32x4*>(base + c * a.sbn)), sp[c]);
+      add8(load16_any(base + c * a.sbn), sp[c]);
   } else if (kk0 < a.k) {
     const int ne = a.k - kk0 < 8 ? (int)(a.k - kk0) : 8;
 #pragma unroll 1
@@ -370,7 +378,8 @@ struct PairE {
   float e0, e1, asq, asum;
 };
 
-template <int NS = SDC_MAX_SPLITS>
+// (MORE: planes past NS are added too)
+template <int NS = SDC_MAX_SPLITS, bool MORE = true>
 __device__ __forceinline__ PairE pair_expected(const TrainArgs& a, int64_t eb, int64_t r, int64_t jb) {
   // E planes row-major ([m][ncols]: plain and signed adjacent) or transposed ([ncols][m]: adjacent rows)
   const float* ep = a.et ? a.E + ((eb * a.splits) * a.ncols + 2 * jb) * a.cv.m + r
@@ -397,11 +406,20 @@ __device__ __forceinline__ PairE pair_expected(const TrainArgs& a, int64_t eb, i
       pe.asq += xa[s];
       pe.asum += xb[s];
     }
+  if (MORE && a.splits > NS) {                   // (a short GEMM's further planes)
+#pragma unroll 8
+    for (int64_t s = NS; s < a.splits; ++s) {
+      pe.e0 += ep[s * estep];
+      pe.e1 += ep[s * estep + (a.et ? a.cv.m : 1)];
+      pe.asq += xp[s * xstep];
+      pe.asum += xp[s * xstep + a.cv.m];
+    }
+  }
   return pe;
 }
 
 // pe: the pair's expected sums when the caller has them (loaded ahead of C), else null
-template <int DT>
+template <int DT, bool MORE = true>
 __device__ __forceinline__ void train_pair(const TrainArgs& a, int64_t p, float pl, float sg, float sq, float l1,
                                            TrainBest& best, int64_t grp = -1, const PairE* pe = nullptr) {
   if (p >= a.cv.npairs) return;
@@ -410,7 +428,7 @@ __device__ __forceinline__ void train_pair(const TrainArgs& a, int64_t p, float 
   const bool last = (jb == a.cv.nb - 1) && (a.cv.rem > 0);
   const float wf = (float)(last ? a.cv.rem : a.cv.bs);
   const int64_t eb = (a.e_batched && grp < 0) ? bc : 0, bbi = grp >= 0 ? grp : (a.b_batched ? bc : 0);
-  const PairE ex = pe ? *pe : pair_expected(a, eb, r, jb);
+  const PairE ex = pe ? *pe : pair_expected<SDC_MAX_SPLITS, MORE>(a, eb, r, jb);
   float e0 = ex.e0, e1 = ex.e1;
   const float asq = ex.asq, asum = ex.asum;
   const float* cs = a.colstat + (bbi * a.ncols + 2 * jb) * 3;
@@ -486,7 +504,8 @@ __device__ __forceinline__ void train_pair(const TrainArgs& a, int64_t p, float 
   best.keyd = k2 > best.keyd ? k2 : best.keyd;
 }
 
-template <int DT>
+// GEN: C has blocks narrower than 128, or more than SDC_MAX_SPLITS planes
+template <int DT, bool GEN>
 __global__ __launch_bounds__(256) void train_score_kernel(TrainArgs a) {
   __shared__ int64_t red_k[4], red_d[4];
   __shared__ int red_u[4];
@@ -498,8 +517,8 @@ __global__ __launch_bounds__(256) void train_score_kernel(TrainArgs a) {
   for (int64_t tile = (int64_t)blockIdx.x * 4 + w; tile < tiles; tile += (int64_t)gridDim.x * 4) {
     const int64_t base = tile * 64;
     float pl, sg, sq, ab;
-    pair_sums<DT>(a.cv, base, lane, sg2, pl, sg, sq, ab);
-    train_pair<DT>(a, base + q * 16 + (lane >> 2), pl, sg, sq, ab, best);
+    pair_sums<DT, GEN>(a.cv, base, lane, sg2, pl, sg, sq, ab);
+    train_pair<DT, GEN>(a, base + q * 16 + (lane >> 2), pl, sg, sq, ab, best);
   }
   int64_t key = wave_max_i64_dpp(best.key), keyd = wave_max_i64_dpp(best.keyd);   // (every lane active)
   int unk = wave_sum_i32_dpp(best.unk);
@@ -545,7 +564,7 @@ __global__ __launch_bounds__(256) void train_score_t_kernel(TrainArgs a) {
   if (a.cv.vec && r0 + 8 <= m) {
 #pragma unroll 8
     for (int c = w; c < wid; c += 4) {
-      const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(base + c * a.cv.sn));
+      const u32x4 v = load16_any(base + c * a.cv.sn);
       const float s = sp[c];
       const float x[8] = {lo_of<DT>(v.x), hi_of<DT>(v.x), lo_of<DT>(v.y), hi_of<DT>(v.y),
                           lo_of<DT>(v.z), hi_of<DT>(v.z), lo_of<DT>(v.w), hi_of<DT>(v.w)};
@@ -641,7 +660,8 @@ constexpr int GSLOT = 64;                         // groups a workgroup gathers 
 // pair's expected sums are loaded before its C.  The waves gather their worst keys and counts per group in LDS (the
 // workgroup's rows span few groups), then one thread per group it touched updates that group's result row: device
 // atomics on one row serialize, so they are made per workgroup, not per wave.  NS: the most split planes added.
-template <int DT, int NS>
+// NARROW: C has blocks narrower than 128.
+template <int DT, int NS, bool NARROW>
 __global__ __launch_bounds__(256) void grouped_score_kernel(TrainArgs a) {
   __shared__ int64_t offs_s[GCAP];
   __shared__ unsigned long long s_key[GSLOT], s_keyd[GSLOT];
@@ -670,9 +690,9 @@ __global__ __launch_bounds__(256) void grouped_score_kernel(TrainArgs a) {
     const int64_t pc = p < a.cv.npairs ? p : a.cv.npairs - 1;
     int64_t bc, r, jb;
     pair_index(a.cv, pc, bc, r, jb);
-    const PairE pe = pair_expected<NS>(a, 0, r, jb);
+    const PairE pe = pair_expected<NS, false>(a, 0, r, jb);
     float pl, sg, sq, ab;
-    pair_sums<DT>(a.cv, base, lane, sg2, pl, sg, sq, ab);
+    pair_sums<DT, NARROW>(a.cv, base, lane, sg2, pl, sg, sq, ab);
     grp = group_of(offs, a.ngroups, r);
     if (grp >= 0) train_pair<DT>(a, p, pl, sg, sq, ab, tb, grp, &pe);
     const int64_t last = base + 63 < a.cv.npairs ? base + 63 : a.cv.npairs - 1;
@@ -781,6 +801,14 @@ struct BConsts {
   const float* b2t;                // the block sums themselves where `parts` are not made yet (frag is), or null
 };
 
+void launch_b_stage(int dtype, const BStageArgs& ba, dim3 grid, hipStream_t stream) {
+  const bool narrow = ba.vec && (ba.rem != 0 || ba.bs != 128);
+  if (dtype == SDC_BF16 && narrow) hipLaunchKernelGGL((b_stage_kernel<SDC_BF16, true>), grid, dim3(256), 0, stream, ba);
+  else if (dtype == SDC_BF16) hipLaunchKernelGGL((b_stage_kernel<SDC_BF16, false>), grid, dim3(256), 0, stream, ba);
+  else if (narrow) hipLaunchKernelGGL((b_stage_kernel<SDC_FP16, true>), grid, dim3(256), 0, stream, ba);
+  else hipLaunchKernelGGL((b_stage_kernel<SDC_FP16, false>), grid, dim3(256), 0, stream, ba);
+}
+
 // The B side: block sums of B and their statistics (b_stage, b_finish), the bias's block sums, and the three parts
 // of the block sums: in fragment order where bc.frag is set (finish_frag) and k-major otherwise (split); both for a
 // layer's constants (bc.frag set, bc.b2t null).  b2t and part are scratch of layout()'s sizes.
@@ -793,8 +821,7 @@ int stage_b(int dtype, const void* B, int64_t sbb, int64_t sbk, int64_t sbn, int
   ba.s_full = s_full; ba.s_last = s_last; ba.B2T = b2t; ba.part = part;
   // B with k-contiguous rows (W.t(), x^T) is read down its columns by b_stage_t_kernel; otherwise across rows
   const bool b_t = sbk == 1 && sbn != 1;
-  if (b_t) ba.vec = (sbn % 8 == 0) && (sbb % 8 == 0) && ((uintptr_t)B % 16 == 0);
-  else ba.vec = sbn == 1 && (sbk % 8 == 0) && (sbb % 8 == 0) && (bs % 8 == 0) && ((uintptr_t)B % 16 == 0);
+  ba.vec = b_t || sbn == 1;
   {
     SdcProf prof("b_stage", stream);
     if (b_t) {
@@ -803,8 +830,7 @@ int stage_b(int dtype, const void* B, int64_t sbb, int64_t sbk, int64_t sbn, int
       else hipLaunchKernelGGL(b_stage_t_kernel<SDC_FP16>, grid, dim3(256), 0, stream, ba);
     } else {
       dim3 grid((unsigned)L.nkc, (unsigned)L.nb, (unsigned)batch_b);
-      if (dtype == SDC_BF16) hipLaunchKernelGGL(b_stage_kernel<SDC_BF16>, grid, dim3(256), 0, stream, ba);
-      else hipLaunchKernelGGL(b_stage_kernel<SDC_FP16>, grid, dim3(256), 0, stream, ba);
+      launch_b_stage(dtype, ba, grid, stream);
     }
     SDC_LAUNCH_CHECK();
   }
@@ -940,7 +966,7 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
   TrainArgs ta{};
   ta.cv.y = (const uint16_t*)C; ta.cv.sb = scb; ta.cv.sm = scm; ta.cv.sn = scn; ta.cv.m = m; ta.cv.nb = L.nb;
   ta.cv.bs = bs; ta.cv.rem = L.rem; ta.cv.npairs = batch_c * m * L.nb; ta.cv.s_full = s_full; ta.cv.s_last = s_last;
-  ta.cv.vec = scn == 1 && (scm % 8 == 0) && (scb % 8 == 0) && (bs % 8 == 0) && ((uintptr_t)C % 16 == 0);
+  ta.cv.vec = scn == 1;
   ta.k = k; ta.splits = splits; ta.nbt = nbt; ta.ncols = L.ncols;
   ta.b_batched = batch_b > 1; ta.e_batched = nbt > 1;
   ta.E = E; ta.XN = XN; ta.colstat = bc.colstat; ta.bmaxf = bc.bmaxf;
@@ -962,29 +988,35 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
     const int64_t tiles = sdc_cdiv(ta.cv.npairs, 64);
     if (sdc_cdiv(tiles, 4) > 0x7FFFFFFF) return SDC_EUNSUPPORTED;
     const unsigned grid = (unsigned)sdc_cdiv(tiles, 4);                // one tile per wave
-    if (ta.splits <= 2) {                                              // (the tall grouped GEMM's two planes)
-      if (dtype == SDC_BF16) hipLaunchKernelGGL((grouped_score_kernel<SDC_BF16, 2>), dim3(grid), dim3(256), 0, stream, ta);
-      else hipLaunchKernelGGL((grouped_score_kernel<SDC_FP16, 2>), dim3(grid), dim3(256), 0, stream, ta);
-    } else if (ta.splits <= 4) {
-      if (dtype == SDC_BF16) hipLaunchKernelGGL((grouped_score_kernel<SDC_BF16, 4>), dim3(grid), dim3(256), 0, stream, ta);
-      else hipLaunchKernelGGL((grouped_score_kernel<SDC_FP16, 4>), dim3(grid), dim3(256), 0, stream, ta);
-    } else {
-      if (dtype == SDC_BF16)
-        hipLaunchKernelGGL((grouped_score_kernel<SDC_BF16, SDC_MAX_SPLITS>), dim3(grid), dim3(256), 0, stream, ta);
-      else
-        hipLaunchKernelGGL((grouped_score_kernel<SDC_FP16, SDC_MAX_SPLITS>), dim3(grid), dim3(256), 0, stream, ta);
-    }
+    auto go = [&](auto dt, auto ns, auto narrow) {
+      hipLaunchKernelGGL((grouped_score_kernel<decltype(dt)::value, decltype(ns)::value, decltype(narrow)::value>),
+                         dim3(grid), dim3(256), 0, stream, ta);
+    };
+    auto with_ns = [&](auto dt, auto narrow) {
+      if (ta.splits <= 2) go(dt, std::integral_constant<int, 2>{}, narrow);          // (the tall grouped GEMM's)
+      else if (ta.splits <= 4) go(dt, std::integral_constant<int, 4>{}, narrow);
+      else go(dt, std::integral_constant<int, SDC_MAX_SPLITS>{}, narrow);
+    };
+    const bool narrow = blocks_narrow(ta.cv);
+    if (dtype == SDC_BF16 && narrow) with_ns(std::integral_constant<int, SDC_BF16>{}, std::true_type{});
+    else if (dtype == SDC_BF16) with_ns(std::integral_constant<int, SDC_BF16>{}, std::false_type{});
+    else if (narrow) with_ns(std::integral_constant<int, SDC_FP16>{}, std::true_type{});
+    else with_ns(std::integral_constant<int, SDC_FP16>{}, std::false_type{});
   } else if (c_t) {
     // C with adjacent rows (y^T): read 512 rows at a time down each column
-    ta.cv.vec = (scn % 8 == 0) && (scb % 8 == 0) && ((uintptr_t)C % 16 == 0);
+    ta.cv.vec = 1;
     dim3 grid((unsigned)sdc_cdiv(m, 512), (unsigned)L.nb, (unsigned)batch_c);
     if (dtype == SDC_BF16) hipLaunchKernelGGL(train_score_t_kernel<SDC_BF16>, grid, dim3(256), 0, stream, ta);
     else hipLaunchKernelGGL(train_score_t_kernel<SDC_FP16>, grid, dim3(256), 0, stream, ta);
   } else {
     const int64_t tiles = sdc_cdiv(ta.cv.npairs, 64);
     const unsigned grid = (unsigned)(sdc_cdiv(tiles, 4) < 1024 ? sdc_cdiv(tiles, 4) : 1024);
-    if (dtype == SDC_BF16) hipLaunchKernelGGL(train_score_kernel<SDC_BF16>, dim3(grid), dim3(256), 0, stream, ta);
-    else hipLaunchKernelGGL(train_score_kernel<SDC_FP16>, dim3(grid), dim3(256), 0, stream, ta);
+    const bool gen = blocks_narrow(ta.cv) || ta.splits > SDC_MAX_SPLITS;
+    const dim3 g1(grid), b1(256);
+    if (dtype == SDC_BF16 && gen) hipLaunchKernelGGL((train_score_kernel<SDC_BF16, true>), g1, b1, 0, stream, ta);
+    else if (dtype == SDC_BF16) hipLaunchKernelGGL((train_score_kernel<SDC_BF16, false>), g1, b1, 0, stream, ta);
+    else if (gen) hipLaunchKernelGGL((train_score_kernel<SDC_FP16, true>), g1, b1, 0, stream, ta);
+    else hipLaunchKernelGGL((train_score_kernel<SDC_FP16, false>), g1, b1, 0, stream, ta);
   }
   SDC_LAUNCH_CHECK();
   return SDC_OK;
@@ -1235,15 +1267,14 @@ extern "C" int sdc_layer_constants(int dtype, const void* W, int64_t swn, int64_
   {
     SdcProf prof("b_stage", stream);
     if (swn != 1) {
-      ba.vec = (swn % 8 == 0) && ((uintptr_t)W % 16 == 0);
+      ba.vec = 1;
       dim3 grid((unsigned)sdc_cdiv(k, 256), (unsigned)L.nb, 1u);
       if (dtype == SDC_BF16) hipLaunchKernelGGL(b_stage_t_kernel<SDC_BF16>, grid, dim3(256), 0, stream, ba);
       else hipLaunchKernelGGL(b_stage_t_kernel<SDC_FP16>, grid, dim3(256), 0, stream, ba);
     } else {                                                            // k == 1: W^T is one contiguous row
-      ba.vec = (bs % 8 == 0) && ((uintptr_t)W % 16 == 0);
+      ba.vec = 1;
       dim3 grid((unsigned)L.nkc, (unsigned)L.nb, 1u);
-      if (dtype == SDC_BF16) hipLaunchKernelGGL(b_stage_kernel<SDC_BF16>, grid, dim3(256), 0, stream, ba);
-      else hipLaunchKernelGGL(b_stage_kernel<SDC_FP16>, grid, dim3(256), 0, stream, ba);
+      launch_b_stage(dtype, ba, grid, stream);
     }
     SDC_LAUNCH_CHECK();
   }

@@ -65,3 +65,23 @@ def test_training_operand_layouts(m, k, n, lb, la, dt):
     ok = z_close(z, o.z.reshape(-1), gemm_slack(o.csb, o.den).reshape(-1))
     assert ok.all(), (np.nonzero(~ok)[0][:5], z[~ok][:5], o.z.reshape(-1)[~ok][:5])
     assert row[2] == 0
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("n,block", [(5, 128), (9, 8), (130, 7), (300, 100), (257, 127), (1000, 128)])
+@pytest.mark.parametrize("batch", [0, 3])
+def test_narrow_blocks(n, block, batch, dt):
+    """Blocks narrower than 128, rows at any 2-byte address, fewer columns than one 16-byte load."""
+    from sdcguard_amd import matmul_zscores
+    m, k = 67, 40
+    g = torch.Generator().manual_seed(n + block)
+    t = torch.bfloat16 if dt == "bf16" else torch.float16
+    lead = (batch,) if batch else ()
+    A, B = torch.randn(*lead, m, k, generator=g).to(t), (torch.randn(*lead, k, n, generator=g) * 0.1).to(t)
+    C = (A.float() @ B.float()).to(t)
+    scores = torch.full((max(1, batch), m, -(-n // min(block, n)), 2), -7.0, device="cuda")
+    matmul_zscores(A.cuda(), B.cuda(), C.cuda(), block=block, scores_out=scores)
+    o = abft.zscores(A.float().numpy(), B.float().numpy(), C.float().numpy(), block=block, dtype=dt, seed=1)
+    z = scores.cpu().numpy().reshape(-1)
+    ok = z_close(z, o.z.reshape(-1), gemm_slack(o.csb, o.den).reshape(-1))
+    assert ok.all(), (np.nonzero(~ok)[0][:5], z[~ok][:5], o.z.reshape(-1)[~ok][:5])
