@@ -366,6 +366,15 @@ int sdc_fingerprint2(const void* bits, int64_t n, int kind, int64_t* out, hipStr
 int sdc_kv_fingerprint(const void* cache, int64_t nblocks, int64_t block_bytes, int64_t words, int word_bytes,
                        const int64_t* ids, int64_t n, int64_t* out, hipStream_t stream);
 
+/* ---- the ledger check of a block table (one entry per logical block): mismatch[i] (a byte, 0 or 1) = known[i] is set,
+ * ids[i] >= 0 and the fingerprint of block ids[i] (zeros for an id >= nblocks) is not expected[i][0..2]; *count = the
+ * number of mismatches.  cache .. word_bytes as sdc_kv_fingerprint; ws: sdc_kv_verify_workspace(n, words, word_bytes)
+ * int64s of scratch. */
+int64_t sdc_kv_verify_workspace(int64_t n, int64_t words, int word_bytes);
+int sdc_kv_verify(const void* cache, int64_t nblocks, int64_t block_bytes, int64_t words, int word_bytes,
+                  const int64_t* ids, int64_t n, const int64_t* expected, const uint8_t* known, uint8_t* mismatch,
+                  int64_t* count, int64_t* ws, int64_t ws_words, hipStream_t stream);
+
 /* ---- sampled attention recompute from a paged KV cache, and the sampled tokens' KV-write check ------------
  * Replaces serve_attn.attn_check_triton (serve_attn.py:574-602) and its two kernels _attn_part / _attn_judge
  * (:335-571); the arithmetic of attn_check_torch (:165-280).  One launch, no host synchronisation.

@@ -413,6 +413,7 @@ __global__ __launch_bounds__(64 * KV_WAVES) void kv_fp3_kernel(KvArgs a, const i
 constexpr int KVM_BYTES = 65536;                 // bytes per block the tables cover (32768 2-byte words)
 constexpr int KVM_STEPS = KVM_BYTES / 32;        // 32-byte steps of a block (one MFMA each)
 constexpr int KVM_ENT = 64;                      // block entries per workgroup: two 32-column tiles per wave
+constexpr int KVM_WGS = 1024;                    // workgroups that fill the chip (four per CU, by registers)
 __device__ __attribute__((aligned(256))) uint8_t kvm_tab[2][KVM_STEPS * 1024];            // [word bytes - 1]
 __device__ __attribute__((aligned(256))) uint64_t kvm_corr[2][2 * (KVM_STEPS + 1)];
 
@@ -495,47 +496,50 @@ __global__ __launch_bounds__(256) void kvm_corr_kernel(uint64_t* corr) {
   }
 }
 
-// Workgroup: entries e0 .. e0 + 63; wave w: the w-th quarter of each block's 128-byte chunks.  Per chunk, each lane
-// loads 8 pieces of 16 bytes (load i: entry 8 i + lane / 8, piece lane % 8: whole lines), flips the low bytes' top
-// bits and stores them to the wave's LDS tile (entry row of 128 bytes, piece j at slot j ^ (row % 8)); then per
-// 32-byte step s and column tile u, lane l reads row 32 u + l % 32, piece 2 s + l / 32 (the B operand) and the
-// MFMA takes the table's step (the A operand) against it.  Chunks alternate between two register sets, the next
-// one's loads issued before the current one is stored.
-template <int WB>
-__global__ __launch_bounds__(256) void kv_mfma_kernel(KvArgs a, const int64_t* ids, const uint8_t* tab,
-                                                      const uint64_t* corr) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds[4][KVM_ENT * 128];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int64_t e0 = (int64_t)blockIdx.x * KVM_ENT;
-  const int64_t chunks = a.words * WB / 128;
-  const int64_t per = (chunks + 3) / 4;
-  const int64_t c0 = w * per < chunks ? w * per : chunks;
-  const int64_t c1 = c0 + per < chunks ? c0 + per : chunks;
-  const uint8_t* src[8];
+// Workgroup (group g, depth part z of Z): entries 64 g .. 64 g + 63, chunks (of 128 bytes) c0 .. c1 of each block, its
+// four waves in turn (wave w: chunks c0 + w, c0 + w + 4, ..., so they read 512 bytes of a block at a time).  The
+// entries that name a block come first in the tile; with at most 32 of them half the loads and products are left out,
+// with none the workgroup ends.  Per chunk, each lane loads 16-byte pieces (load i: row 8 i + lane / 8, piece lane % 8:
+// whole lines), flips the low bytes' top bits and stores them to the wave's LDS tile (row of 128 bytes, piece j at
+// slot j ^ (row % 8)); then per 32-byte step s and column tile u, lane l reads row 32 u + l % 32, piece 2 s + l / 32
+// (the B operand) and the MFMA takes the table's step (the A operand) against it.  Chunks alternate between two
+// register sets, the next one's loads issued before the current one is stored.
+// Bound by memory, so the depth is split until the chip is full: the entries alone gave 128 workgroups for a table of
+// 64 x 128 entries, whose 5120 blocks of 64 KiB (335 MB) took 136 us; over 8 parts they take 73 us (4.6 TB/s).  Part z runs on XCD z % 8 when Z is a multiple of 8 (dispatch is
+// round-robin), so an XCD's L2 holds its own parts of the weight table.
+// The workgroup's sums go to plane z of `planes` ([Z][n][3], only the entries that name a block), or are added to
+// a.out when there is none.
+struct KvmGeom {
+  int64_t chunks, per;             // chunks of a block, chunks per part
+  int64_t parts;                   // Z
+  int64_t* planes;
+  int64_t* count;                  // set to zero when not null (kv_compare_kernel counts into it)
+};
+
+__device__ __forceinline__ int64_t kv_entry(const KvArgs& a, const int64_t* ids, int64_t ent) {
+  int64_t blk = -1;
+  if (ent < a.n) blk = ids ? ids[ent] : ent;
+  return blk >= 0 && blk < a.nblocks ? blk : -1;
+}
+
+template <int WB, int NU>          // NU: column tiles of 32 entries
+__device__ __forceinline__ void kvm_chunks(const KvArgs& a, const int64_t* rowblk, uint8_t* L, const uint8_t* tab,
+                                           int64_t c0, int64_t c1, i32x16 (&acc)[2]) {
+  const int lane = threadIdx.x & 63;
+  constexpr int NL = 4 * NU;
+  const uint8_t* src[NL];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int64_t ent = e0 + 8 * i + (lane >> 3);
-    int64_t blk = -1;
-    if (ent < a.n) blk = ids ? ids[ent] : ent;
-    const bool live = blk >= 0 && blk < a.nblocks;
-    src[i] = a.cache + (live ? blk : 0) * a.block_bytes + 16 * (lane & 7);
-  }
-  uint8_t* const L = lds[w];
-  i32x16 acc[2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[u][e] = 0;
+  for (int i = 0; i < NL; ++i) src[i] = a.cache + rowblk[8 * i + (lane >> 3)] * a.block_bytes + 16 * (lane & 7);
   auto load = [&](int64_t c, u32x4* d, i32x4* tf) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) d[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src[i] + 128 * c));
+    for (int i = 0; i < NL; ++i) d[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src[i] + 128 * c));
 #pragma unroll
     for (int s = 0; s < 4; ++s) tf[s] = *reinterpret_cast<const i32x4*>(tab + (4 * c + s) * 1024 + 16 * lane);
   };
   const int wslot = (lane & 7) ^ (lane >> 3);                  // load i's piece lane % 8 of row 8 i + lane / 8
   auto process = [&](const u32x4* d, const i32x4* tf) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < NL; ++i) {
       // 2-byte words: the low bytes' top bits flipped (lo - 128); 1-byte words as they are
       const u32x4 x = WB == 2 ? d[i] ^ u32x4{0x00800080u, 0x00800080u, 0x00800080u, 0x00800080u} : d[i];
       *reinterpret_cast<u32x4*>(L + (8 * i + (lane >> 3)) * 128 + 16 * wslot) = x;
@@ -543,25 +547,63 @@ __global__ __launch_bounds__(256) void kv_mfma_kernel(KvArgs a, const int64_t* i
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < NU; ++u) {
         const int row = 32 * u + (lane & 31), piece = 2 * s + (lane >> 5);
         const i32x4 b = *reinterpret_cast<const i32x4*>(L + row * 128 + 16 * (piece ^ (row & 7)));
         acc[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(tf[s], b, acc[u], 0, 0, 0);
       }
   };
   if (c0 < c1) {
-    u32x4 da[8], db[8];
+    u32x4 da[NL], db[NL];
     i32x4 ta[4], tb[4];
     load(c0, da, ta);
-    for (int64_t c = c0; c < c1; c += 2) {
-      if (c + 1 < c1) load(c + 1, db, tb);
+    for (int64_t c = c0; c < c1; c += 8) {
+      if (c + 4 < c1) load(c + 4, db, tb);
       process(da, ta);
-      if (c + 1 >= c1) break;
-      if (c + 2 < c1) load(c + 2, da, ta);
+      if (c + 4 >= c1) break;
+      if (c + 8 < c1) load(c + 8, da, ta);
       process(db, tb);
     }
   }
-  // lane l holds column (entry) 32 u + l % 32 of tile u, rows 8 (e / 4) + 4 (l / 32) + e % 4 of its 16 values
+}
+
+template <int WB>
+__global__ __launch_bounds__(256) void kv_mfma_kernel(KvArgs a, const int64_t* ids, const uint8_t* tab,
+                                                      const uint64_t* corr, KvmGeom g) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[4][KVM_ENT * 128];
+  __shared__ int64_t rowblk[KVM_ENT];            // row r of the tile: its block
+  __shared__ int rowent[KVM_ENT];                // and its entry in the group
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  if (g.count && blockIdx.x == 0 && t == 0) *g.count = 0;
+  const int64_t z = blockIdx.x % g.parts, e0 = blockIdx.x / g.parts * KVM_ENT;
+  const int64_t blk = kv_entry(a, ids, e0 + lane);
+  const uint64_t live = __builtin_amdgcn_ballot_w64(blk >= 0);
+  const int nlive = __builtin_popcountll(live);
+  if (nlive == 0) return;
+  if (w == 0) {
+    const uint64_t below = (1ull << lane) - 1ull;
+    // (rows past the live ones read entry `first`'s block once more; their sums are not used)
+    const int row = blk >= 0 ? __builtin_popcountll(live & below) : nlive + __builtin_popcountll(~live & below);
+    const int first = __builtin_ctzll(live);
+    const int64_t fb = ((int64_t)__builtin_amdgcn_readlane((int)(blk >> 32), first) << 32) |
+                       (uint32_t)__builtin_amdgcn_readlane((int)blk, first);
+    rowblk[row] = blk >= 0 ? blk : fb;
+    rowent[row] = lane;
+  }
+  __syncthreads();
+  const int64_t c0 = z * g.per < g.chunks ? z * g.per : g.chunks;
+  const int64_t c1 = c0 + g.per < g.chunks ? c0 + g.per : g.chunks;
+  i32x16 acc[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[u][e] = 0;
+  if (nlive <= 32) kvm_chunks<WB, 1>(a, rowblk, lds[w], tab, c0 + w, c1, acc);
+  else kvm_chunks<WB, 2>(a, rowblk, lds[w], tab, c0 + w, c1, acc);
+  // lane l holds column (row of the tile) 32 u + l % 32, rows 8 (e / 4) + 4 (l / 32) + e % 4 of its 16 values; the
+  // workgroup's eight partial sums of a row (four waves, two lane halves) are added over LDS
+  __syncthreads();
+  uint64_t* red = reinterpret_cast<uint64_t*>(lds);           // [component][wave and half][row]
   const int h = lane >> 5;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
@@ -575,21 +617,69 @@ __global__ __launch_bounds__(256) void kv_mfma_kernel(KvArgs a, const int64_t* i
       else if (r == 16) v0 += x;
       else if (r == 17) v0 += x << 8;
     }
-    if (WB == 2 && h == 0) {
-      v0 += (uint64_t)(128 * 64) * (uint64_t)(c1 - c0);
-      v1 += corr[4 * c1] - corr[4 * c0];
-      v2 += corr[(KVM_STEPS + 1) + 4 * c1] - corr[(KVM_STEPS + 1) + 4 * c0];
-    }
-    const int64_t ent = e0 + 32 * u + (lane & 31);
-    int64_t blk = -1;
-    if (ent < a.n) blk = ids ? ids[ent] : ent;
-    if (blk >= 0 && blk < a.nblocks && c0 < c1) {
-      int64_t* o = a.out + 3 * ent;
-      if (h == 0) atomicAdd((unsigned long long*)o, (unsigned long long)v0);
-      atomicAdd((unsigned long long*)(o + 1), (unsigned long long)v1);
-      atomicAdd((unsigned long long*)(o + 2), (unsigned long long)v2);
-    }
+    const int at = (2 * w + h) * KVM_ENT + 32 * u + (lane & 31);
+    red[at] = v0;
+    red[8 * KVM_ENT + at] = v1;
+    red[16 * KVM_ENT + at] = v2;
   }
+  __syncthreads();
+  const int row = t % KVM_ENT, comp = t / KVM_ENT;
+  if (comp < 3 && row < nlive) {
+    uint64_t v = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v += red[(8 * comp + q) * KVM_ENT + row];
+    if (WB == 2) {
+      if (comp == 0) v += (uint64_t)(128 * 64) * (uint64_t)(c1 - c0);
+      else v += corr[(comp - 1) * (KVM_STEPS + 1) + 4 * c1] - corr[(comp - 1) * (KVM_STEPS + 1) + 4 * c0];
+    }
+    const int64_t ent = e0 + rowent[row];
+    if (g.planes) g.planes[(z * a.n + ent) * 3 + comp] = (int64_t)v;
+    else atomicAdd((unsigned long long*)(a.out + 3 * ent + comp), (unsigned long long)v);
+  }
+}
+
+// The number of depth parts: as many workgroups as fit the chip at once, each wave at least four chunks (twice and
+// four times as many workgroups: 5 % and 2 % slower, each with fewer bytes per weight-table load and prologue)
+int64_t kvm_parts(int64_t n, int64_t chunks) {
+  const int64_t groups = sdc_cdiv(n, KVM_ENT);
+  int64_t parts = 1;
+  while (parts < 32 && groups * parts < KVM_WGS && chunks >= 2 * parts * 16) parts *= 2;
+  return parts;
+}
+
+// mismatch[i] = known[i] and entry i names a block slot (id >= 0) and its fingerprint (the planes' sum; zero for an id
+// past the cache) differs from expected[i]; *count += the mismatches
+__global__ __launch_bounds__(256) void kv_compare_kernel(const int64_t* planes, int64_t nplanes, const int64_t* ids,
+                                                         int64_t n, int64_t nblocks, const int64_t* expected,
+                                                         const uint8_t* known, uint8_t* mismatch, int64_t* count) {
+  __shared__ int cnt[4];
+  const int t = threadIdx.x;
+  const int64_t i = (int64_t)blockIdx.x * 256 + t;
+  bool bad = false;
+  if (i < n) {
+    const int64_t id = ids[i];
+    if (id >= 0 && known[i]) {
+      int64_t v[3] = {0, 0, 0};
+      if (id < nblocks)
+        for (int64_t z = 0; z < nplanes; ++z)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) v[c] += planes[(z * n + i) * 3 + c];
+      bad = v[0] != expected[3 * i] || v[1] != expected[3 * i + 1] || v[2] != expected[3 * i + 2];
+    }
+    mismatch[i] = bad ? 1 : 0;
+  }
+  const uint64_t bits = __builtin_amdgcn_ballot_w64(bad);
+  if ((t & 63) == 0) cnt[t >> 6] = __builtin_popcountll(bits);
+  __syncthreads();
+  if (t == 0) {
+    const int c = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+    if (c) atomicAdd((unsigned long long*)count, (unsigned long long)c);
+  }
+}
+
+__global__ __launch_bounds__(256) void kv_zero_kernel(int64_t* p, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0;
 }
 
 constexpr int KVM_MAXDEV = 64;
@@ -675,6 +765,50 @@ extern "C" int sdc_fingerprint2(const void* bits, int64_t n, int kind, int64_t* 
   return SDC_OK;
 }
 
+namespace {
+
+// The fingerprints of a cache's blocks, added to a.out or, where there is room for planes, stored to them (*planes_used
+// of them; the vector kernel adds to plane 0, which is cleared here first), and *count cleared
+int kv_fingerprints(KvArgs a, int word_bytes, int64_t* planes, int64_t* planes_used, int64_t* count,
+                    hipStream_t stream) {
+  a.vec = (a.block_bytes % 16 == 0) && ((uintptr_t)a.cache % 16 == 0);
+  const int64_t* ids = a.ids;
+  // words in whole 128-byte chunks, aligned, within the tables: the MFMA kernel
+  const uint8_t* tab = nullptr;
+  const uint64_t* corr = nullptr;
+  const int64_t wbytes = a.words * word_bytes;
+  if (a.vec && wbytes % 128 == 0 && wbytes <= KVM_BYTES && kvm_tables(stream, word_bytes, &tab, &corr)) {
+    const int64_t chunks = wbytes / 128, parts = kvm_parts(a.n, chunks);
+    const KvmGeom g{chunks, sdc_cdiv(chunks, parts), parts, planes, count};
+    if (planes) *planes_used = parts;
+    SdcProf prof("kv_fingerprint", stream);
+    const dim3 grid((unsigned)(sdc_cdiv(a.n, KVM_ENT) * parts));
+    if (word_bytes == 2) hipLaunchKernelGGL(kv_mfma_kernel<2>, grid, dim3(256), 0, stream, a, ids, tab, corr, g);
+    else hipLaunchKernelGGL(kv_mfma_kernel<1>, grid, dim3(256), 0, stream, a, ids, tab, corr, g);
+    SDC_LAUNCH_CHECK();
+    return SDC_OK;
+  }
+  if (planes) {
+    *planes_used = 1;
+    a.out = planes;
+    hipLaunchKernelGGL(kv_zero_kernel, dim3((unsigned)sdc_cdiv(3 * a.n, 256)), dim3(256), 0, stream, planes, 3 * a.n);
+    hipLaunchKernelGGL(kv_zero_kernel, dim3(1), dim3(256), 0, stream, count, (int64_t)1);
+  }
+  const int64_t gx = sdc_cdiv(sdc_cdiv(a.words, KV_SLICE), KV_WAVES);      // workgroups of KV_WAVES wave slices
+  int64_t gy = sdc_cdiv(2048, gx);
+  if (gy > sdc_cdiv(a.n, KV_UNROLL)) gy = sdc_cdiv(a.n, KV_UNROLL);
+  if (gy > 65535) gy = 65535;
+  SdcProf prof("kv_fingerprint", stream);
+  if (word_bytes == 2)
+    hipLaunchKernelGGL(kv_fp3_kernel<2>, dim3((unsigned)gx, (unsigned)gy), dim3(64 * KV_WAVES), 0, stream, a, ids);
+  else
+    hipLaunchKernelGGL(kv_fp3_kernel<1>, dim3((unsigned)gx, (unsigned)gy), dim3(64 * KV_WAVES), 0, stream, a, ids);
+  SDC_LAUNCH_CHECK();
+  return SDC_OK;
+}
+
+}  // namespace
+
 // out[i][0..2] (int64, zeroed by the caller) += fp3 of block ids[i] (or block i) of a paged cache of int16 words
 // (word_bytes 2) or int8 words (1): block b holds `words` words at cache + b * block_bytes, its positions numbered
 // from 0.  Entries whose id is negative or >= nblocks are left as they are.
@@ -684,29 +818,32 @@ extern "C" int sdc_kv_fingerprint(const void* cache, int64_t nblocks, int64_t bl
   if (word_bytes != 1 && word_bytes != 2) return SDC_EINVAL;
   if (!cache || !out || nblocks < 1 || words < 1 || n < 0 || block_bytes < words * word_bytes) return SDC_EINVAL;
   if (n == 0) return SDC_OK;
-  KvArgs a{(const uint8_t*)cache, block_bytes, words, nblocks, ids, n, out,
-           (block_bytes % 16 == 0) && ((uintptr_t)cache % 16 == 0)};
-  const int64_t gx = sdc_cdiv(sdc_cdiv(words, KV_SLICE), KV_WAVES);      // workgroups of KV_WAVES wave slices
-  int64_t gy = sdc_cdiv(2048, gx);
-  if (gy > sdc_cdiv(n, KV_UNROLL)) gy = sdc_cdiv(n, KV_UNROLL);
-  if (gy > 65535) gy = 65535;
-  // words in whole 128-byte chunks, aligned, within the tables: the MFMA kernel
-  const uint8_t* tab = nullptr;
-  const uint64_t* corr = nullptr;
-  const int64_t wbytes = words * word_bytes;
-  if (a.vec && wbytes % 128 == 0 && wbytes <= KVM_BYTES && kvm_tables(stream, word_bytes, &tab, &corr)) {
-    SdcProf prof("kv_fingerprint", stream);
-    const dim3 grid((unsigned)sdc_cdiv(n, KVM_ENT));
-    if (word_bytes == 2) hipLaunchKernelGGL(kv_mfma_kernel<2>, grid, dim3(256), 0, stream, a, ids, tab, corr);
-    else hipLaunchKernelGGL(kv_mfma_kernel<1>, grid, dim3(256), 0, stream, a, ids, tab, corr);
-    SDC_LAUNCH_CHECK();
-    return SDC_OK;
-  }
-  SdcProf prof("kv_fingerprint", stream);
-  if (word_bytes == 2)
-    hipLaunchKernelGGL(kv_fp3_kernel<2>, dim3((unsigned)gx, (unsigned)gy), dim3(64 * KV_WAVES), 0, stream, a, ids);
-  else
-    hipLaunchKernelGGL(kv_fp3_kernel<1>, dim3((unsigned)gx, (unsigned)gy), dim3(64 * KV_WAVES), 0, stream, a, ids);
+  const KvArgs a{(const uint8_t*)cache, block_bytes, words, nblocks, ids, n, out, 0};
+  return kv_fingerprints(a, word_bytes, nullptr, nullptr, nullptr, stream);
+}
+
+// int64s of scratch sdc_kv_verify needs for n entries of blocks of `words` words
+extern "C" int64_t sdc_kv_verify_workspace(int64_t n, int64_t words, int word_bytes) {
+  if (n < 1 || words < 1) return 0;
+  return 3 * n * kvm_parts(n, words * word_bytes / 128);
+}
+
+// The ledger check of a block table: mismatch[i] (1 byte) = known[i] and ids[i] >= 0 and block ids[i]'s fingerprint is
+// not expected[i][0..2]; *count = the number of mismatches.  Two launches (four on the vector kernel), the fingerprints in planes of ws.
+extern "C" int sdc_kv_verify(const void* cache, int64_t nblocks, int64_t block_bytes, int64_t words, int word_bytes,
+                             const int64_t* ids, int64_t n, const int64_t* expected, const uint8_t* known,
+                             uint8_t* mismatch, int64_t* count, int64_t* ws, int64_t ws_words, hipStream_t stream) {
+  SDC_CLEAR_ERRORS();
+  if (word_bytes != 1 && word_bytes != 2) return SDC_EINVAL;
+  if (!cache || !ids || !expected || !known || !mismatch || !count || !ws || nblocks < 1 || words < 1 || n < 1 ||
+      block_bytes < words * word_bytes || ws_words < sdc_kv_verify_workspace(n, words, word_bytes))
+    return SDC_EINVAL;
+  const KvArgs a{(const uint8_t*)cache, block_bytes, words, nblocks, ids, n, nullptr, 0};
+  int64_t planes = 0;
+  const int rc = kv_fingerprints(a, word_bytes, ws, &planes, count, stream);
+  if (rc != SDC_OK) return rc;
+  hipLaunchKernelGGL(kv_compare_kernel, dim3((unsigned)sdc_cdiv(n, 256)), dim3(256), 0, stream, ws, planes, ids, n,
+                     nblocks, expected, known, mismatch, count);
   SDC_LAUNCH_CHECK();
   return SDC_OK;
 }

@@ -189,3 +189,40 @@ def test_qwen3_like_cache_28_layers_4096_blocks():
     r = led.verify(bt).read()
     want = sorted(tuple(x) for x in (bt == blk).nonzero().cpu().tolist())
     assert sorted(r["entries"]) == want
+
+
+@pytest.mark.parametrize("words,dtype,rows,width", [
+    (64, torch.int16, 1, 1),            # one chunk: one wave of one workgroup
+    (2048 + 64, torch.int16, 5, 13),    # 33 chunks over two depth parts (the second shorter), 65 entries
+    (32768, torch.int16, 3, 43),        # the table's limit over 32 parts; groups of 64 with fewer than 33 live
+    (65536, torch.int8, 2, 64),         # 1-byte words at the limit
+    (1000, torch.int16, 4, 20),         # not whole chunks: the vector kernel
+])
+def test_ledger_verify_matches_fingerprints_entry_by_entry(words, dtype, rows, width):
+    """The fused check (fingerprints in planes, compared and counted on the device) against the fingerprints of the
+    blocks one by one, with no-block entries (whole groups of 64 too), ids past the cache, entries never recorded,
+    repeated blocks and rows whose values changed."""
+    from sdcguard_amd.kv import KVLedger, block_fingerprints
+    info = torch.iinfo(dtype)
+    g = torch.Generator(device="cuda").manual_seed(words)
+    cache = torch.randint(info.min, info.max + 1, (23, words), generator=g, device="cuda", dtype=torch.int32).to(dtype)
+    cache[0], cache[1] = info.min, info.max
+    bt = torch.randint(-6, 23, (rows, width), generator=g, device="cuda")
+    if bt.numel() > 64:
+        bt.view(-1)[:64] = -1                                # the first group names no block
+    bt.view(-1)[-1] = 1
+    led = KVLedger(cache, rows, width)
+    known = torch.rand(rows, width, generator=g, device="cuda") < 0.8
+    known.view(-1)[-1] = True
+    led.record(bt, known)
+    now = bt.clone()
+    now.view(-1)[:: 7] = torch.randint(-1, 26, now.view(-1)[:: 7].shape, generator=g, device="cuda")
+    cache[5, words - 1] ^= 1
+    cache[1, words // 2] ^= 64
+    fp = block_fingerprints(cache, now).view(rows, width, 3)
+    want = led.known & (now >= 0) & (fp != led.expected).any(-1)
+    for table in (now, now.to(torch.int32), now.t().contiguous().t()):
+        got = led.verify(table)
+        assert torch.equal(got.mismatch, want) and int(got.count) == int(want.sum()) > 0
+    one = led.verify(now[:1])                                # a row against every row of the ledger (broadcast)
+    assert one.mismatch.shape == (rows, width)
