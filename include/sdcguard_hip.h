@@ -431,7 +431,7 @@ int sdc_attn_check_noalloc(int dtype, const void* q, int64_t sqt, int64_t sqh, c
  * "serve_score", "b_stage", "b_finish", "split", "train_gemm", "train_score" (also the grouped check's),
  * "col_gemm", "xstage", "xfinish", "row_gemm", "ypass" (sdc_linear_check), "quant_gemm_i8", "quant_gemm_fp8",
  * "quant_score_i8", "quant_score_fp8", "fingerprint3", "fingerprint2", "kv_fingerprint", "attn_check", "acc_bsums",
- * "acc_finish", "acc_anorm", "acc_gemm", "acc_score" (sdc_matmul_check_acc, sdc_matmul_check_acc_stats),
+ * "acc_gemm", "acc_score" (sdc_matmul_check_acc, sdc_matmul_check_acc_stats),
  * "fused_pack", "fused_side", "fused_mm", "fused_mm_checked" (sdc_fused_mm, sdc_fused_mm_checked), "fp8q_amax",
  * "fp8q_judge" (sdc_fp8_quant_check), "moe_up", "moe_act", "moe_down", "moe_compare" (sdc_moe_check), "route_check" (sdc_route_check). */
 int sdc_profile_enable(int on);

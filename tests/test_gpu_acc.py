@@ -110,6 +110,35 @@ def test_precise_kernel_matches_oracle(dt, m, k, n, bias, batch, nfma):
     assert res.row == m // 2 and res.col_block == (n - 3) // 128
 
 
+@pytest.mark.parametrize("m,k,n,a_at,b_at", [
+    (1, 1, 1, "rows", "rows"),                  # element loads everywhere: fewer than 8 columns and depths
+    (33, 7, 129, "odd", "depth"),               # 3 rows past a 32-row tile; a one-column block; depths below 8
+    (129, 33, 7, "rows", "rows"),               # one row past a workgroup; one depth past a segment
+    (65, 100, 577, "odd", "depth"),             # last segment of 4 depths; 5 blocks: one tile of 16 columns
+    (40, 95, 2305, "odd", "odd"),               # 19 blocks (the last one column wide): three tiles
+    (200, 257, 4100, "strided", "strided"),     # 33 blocks: five tiles over two groups; no unit stride
+    (96, 2047, 1200, "depth", "rows"),          # A depth-strided; 31 depth parts
+])
+def test_precise_kernel_edges_and_layouts(m, k, n, a_at, b_at):
+    """Tile, segment and part edges over the layouts of A and B that take loads of their own: rows at 16-byte steps
+    (rows), at odd ones (odd), transposed (depth) and with no unit stride (strided)."""
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+
+    def put(r, c, at, std):
+        if at == "depth":
+            return (torch.randn(c, r, device="cuda", generator=g) * std).bfloat16().t()
+        pad, step = {"rows": (0, 1), "odd": (1 + c % 2, 1), "strided": (0, 2)}[at]
+        return (torch.randn(r, step * c + pad, device="cuda", generator=g) * std).bfloat16()[:, pad::step][:, :c]
+    A, B = put(m, k, a_at, 1.0), put(k, n, b_at, 0.05)
+    C = (A.double() @ B.double()).float()
+    C[m // 2, n // 2] += 1.0
+    zs, res = _scores(A, B, C, nfma=16)
+    o = oacc.acc_zscores(A.float().cpu().numpy(), B.float().cpu().numpy(), C.cpu().numpy(), None, nfma=16, seed=1)
+    ok = z_close(zs.reshape(-1), o.z.reshape(-1))
+    assert ok.all(), (np.nonzero(~ok.reshape(-1))[0][:5], zs.reshape(-1)[~ok][:5], o.z.reshape(-1)[~ok][:5])
+    assert res.row == m // 2 and res.col_block == (n // 2) // 128
+
+
 def test_empty_products_and_huge_cancelling_outputs():
     from sdcguard_amd.checksum import _signs, check_matmul_acc
     for m, k, n in ((0, 64, 256), (8, 64, 0), (8, 0, 256)):
