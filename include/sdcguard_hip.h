@@ -246,6 +246,17 @@ int sdc_parts_fragments(const void* parts, int64_t spc, int64_t N, int64_t k, vo
  * k a multiple of 64; out: sdc_digit_fragments_bytes(N, k) bytes, 8-byte aligned. */
 int64_t sdc_digit_fragments_bytes(int64_t N, int64_t k);
 int sdc_digit_fragments(const void* parts, int64_t spc, int64_t N, int64_t k, void* out, hipStream_t stream);
+
+/* ---- a quantized weight's constants for sdc_quant_check (the checksums of B in modes.py:231-291).  B: k x n bytes,
+ * element strides (sbk, sbn); blocks of `block` <= 128 columns, nb = ceil(n / block); sign_table as sdc_quant_check.
+ *   kind 0 (int8): parts (2, 2 nb, k rounded up to even) int8, the block sums' base-128 digits; no sb.  (Every sum
+ *     splits unless it is 16384: 128 entries of -128 under a pattern of -1 only, which the caller refuses.)
+ *   kind 1 (fp8 e4m3): parts (3, 2 nb, k) bf16 of the scaled sums (sb: n float64 column scales, or NULL for 1), bfrob
+ *     (nb) and bcol (n) fp32; ws: sdc_quant_constants_workspace(kind, k, n) bytes. */
+int64_t sdc_quant_constants_workspace(int kind, int64_t k, int64_t n);
+int sdc_quant_constants(int kind, const void* B, int64_t sbk, int64_t sbn, int64_t k, int64_t n, int64_t block,
+                        const float* sign_table, const double* sb, void* parts, float* bfrob, float* bcol, void* ws,
+                        int64_t ws_bytes, hipStream_t stream);
 int sdc_linear_check(int dtype, const void* x, int64_t sxm, const void* W, int64_t swn, const void* y, int64_t sym,
                      const void* bias, int64_t m, int64_t k, int64_t n, const void* parts, int64_t spc,
                      const void* parts_frag, const float* block_consts, const float* w_norms, const float* sign_table, int64_t* state,
@@ -430,7 +441,7 @@ int sdc_attn_check_noalloc(int dtype, const void* q, int64_t sqt, int64_t sqh, c
  * them and sums the durations of one kernel: "expected_gemm" (serving GEMM), "serve_fused", "serve_sums",
  * "serve_score", "b_stage", "b_finish", "split", "train_gemm", "train_score" (also the grouped check's),
  * "col_gemm", "xstage", "xfinish", "row_gemm", "ypass" (sdc_linear_check), "quant_gemm_i8", "quant_gemm_fp8",
- * "quant_score_i8", "quant_score_fp8", "fingerprint3", "fingerprint2", "kv_fingerprint", "attn_check", "acc_bsums",
+ * "quant_score_i8", "quant_score_fp8", "quant_consts", "fingerprint3", "fingerprint2", "kv_fingerprint", "attn_check", "acc_bsums",
  * "acc_gemm", "acc_score" (sdc_matmul_check_acc, sdc_matmul_check_acc_stats),
  * "fused_pack", "fused_side", "fused_mm", "fused_mm_checked" (sdc_fused_mm, sdc_fused_mm_checked), "fp8q_amax",
  * "fp8q_judge" (sdc_fp8_quant_check), "moe_up", "moe_act", "moe_down", "moe_compare" (sdc_moe_check), "route_check" (sdc_route_check). */

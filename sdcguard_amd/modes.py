@@ -65,10 +65,12 @@ class QuantChecksums:
         if B.dim() != 2:
             raise ValueError("B must be (k, n)")
         k, n = B.shape
+        if B.dtype == torch.int8 and sb is not None:
+            raise ValueError("int8 check: no scales (the accumulator itself is checked, exactly)")
+        if B.is_cuda and k and n and 1 <= block <= BLOCK and _device_constants(B, sb, block):
+            return cls._make_on_device(B, sb, block)
         W = _block_weights(n, block, B.device)
         if B.dtype == torch.int8:
-            if sb is not None:
-                raise ValueError("int8 check: no scales (the accumulator itself is checked, exactly)")
             B2 = B.double() @ W                                   # exact: |B2| <= 128 * 128 = 16384
             # two base-128 digits, B2 = 128 hi + lo with hi in [-128, 127]: |lo| <= 64 except for sums in
             # [16320, 16383] (-128 entries laid against the sign pattern), whose lo takes 64..127.  +16384 would
@@ -91,6 +93,37 @@ class QuantChecksums:
             sq = torch.nn.functional.pad(Bs.pow(2).sum(0), (0, pad)).view(nb, block).sum(1)
             return cls("fp8", k, n, block, parts.contiguous(), sq.sqrt().float(), Bs.pow(2).sum(0).sqrt().float())
         raise ValueError(f"unsupported weight dtype {B.dtype} (int8 or float8_e4m3fn)")
+
+    @classmethod
+    def _make_on_device(cls, B: torch.Tensor, sb: Optional[torch.Tensor], block: int) -> "QuantChecksums":
+        """sdc_quant_constants: one pass over B (the products with the pattern in float64, by torch, took a dozen)."""
+        from . import _lib
+        k, n = B.shape
+        nb, dev = -(-n // block), B.device
+        i8 = B.dtype == torch.int8
+        L, tab = _lib.lib(), sign_table(dev)
+        bfrob = bcol = ws = scales = None
+        if i8:
+            parts = torch.empty(2, 2 * nb, k + k % 2, dtype=torch.int8, device=dev)
+        else:
+            parts = torch.empty(3, 2 * nb, k, dtype=torch.bfloat16, device=dev)
+            bfrob = torch.empty(nb, dtype=torch.float32, device=dev)
+            bcol = torch.empty(n, dtype=torch.float32, device=dev)
+            ws = torch.empty(int(L.sdc_quant_constants_workspace(1, k, n)), dtype=torch.uint8, device=dev)
+            scales = None if sb is None else sb.double().reshape(n).contiguous()
+        _lib.check(L.sdc_quant_constants(0 if i8 else 1, B.data_ptr(), B.stride(0), B.stride(1), k, n, block,
+                                         tab.data_ptr(), _lib.ptr(scales) or None, parts.data_ptr(),
+                                         _lib.ptr(bfrob) or None, _lib.ptr(bcol) or None, _lib.ptr(ws) or None,
+                                         0 if ws is None else ws.numel(), _lib.stream_of(B)), "sdc_quant_constants")
+        return cls("int8" if i8 else "fp8", k, n, block, parts, bfrob, bcol)
+
+
+def _device_constants(B: torch.Tensor, sb: Optional[torch.Tensor], block: int) -> bool:
+    """Whether sdc_quant_constants makes this weight's constants.  A signed int8 sum reaches 16384, which does not split
+    and is refused, only under a width-128 pattern without a +1 entry: such a pattern keeps the path that looks at the sums."""
+    if B.dtype == torch.float8_e4m3fn:
+        return sb is None or (sb.device == B.device and sb.numel() == B.shape[1])
+    return B.dtype == torch.int8 and (block < BLOCK or bool((sign_table("cpu").view(128, 128)[BLOCK - 1] > 0).any()))
 
 
 @dataclass

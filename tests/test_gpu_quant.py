@@ -431,3 +431,47 @@ def test_quant_row_checks_at_2048x7168x4096():
     c[77, 4000] += 4 * C[:128, 4000].pow(2).mean().sqrt()
     res = modes.judge_rows("fp8", Aq, Bq, c, sa=sa, sb=sb)
     assert res["wrong_blocks"] == 1 and (res["row"], res["block"]) == (4000, 0), res
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp8"])
+@pytest.mark.parametrize("k,n,layout,block", [
+    (1, 1, "rows", 128),                # one value
+    (63, 129, "rows", 128),             # a short slice; a one-column block; rows at odd bytes
+    (65, 250, "columns", 128),          # a slice of one depth; columns at odd bytes; a block 122 wide
+    (130, 300, "strided", 128),         # no unit stride
+    (97, 40, "rows", 16),               # narrower blocks
+])
+def test_constants_made_on_the_device(kind, k, n, layout, block):
+    """sdc_quant_constants against the sums in float64 on the CPU: int8 digits exactly (the depth's zero digit too), fp8
+    parts to bf16's part of their column's sum, norms to fp32 rounding; values at the type's extremes."""
+    from sdcguard_amd import modes
+    from sdcguard_amd.checksum import sign_table
+    g = torch.Generator().manual_seed(k + n)
+    if kind == "int8":
+        B = torch.randint(-128, 128, (k, n), generator=g, dtype=torch.int32)
+        B[0] = -128
+        B, sb = B.to(torch.int8), None
+    else:
+        B = (torch.randn(k, n, generator=g) * 100).clamp(-448, 448)
+        B[0], sb = 448.0, 10.0 ** (torch.rand(n, generator=g) * 4 - 3)
+        B = B.to(torch.float8_e4m3fn)
+    raw = B.view(torch.uint8)
+    dev = {"rows": lambda: raw.cuda(), "columns": lambda: raw.t().contiguous().cuda().t(),
+           "strided": lambda: raw.repeat_interleave(2, 1).cuda()[:, ::2]}[layout]().view(B.dtype)
+    c = modes.QuantChecksums.make(dev, None if sb is None else sb.cuda(), block)
+    Bd = B.float().double() * (1.0 if sb is None else sb.double())
+    tab = sign_table("cpu").double().view(128, 128)
+    want = []
+    for lo in range(0, n, block):
+        v = Bd[:, lo:lo + block]
+        want += [v.sum(1), v @ tab[v.shape[1] - 1, :v.shape[1]]]
+    want = torch.stack(want)                                              # (2 nb, k)
+    parts = c.parts.cpu().double()
+    if kind == "int8":
+        assert torch.equal((128 * parts[0] + parts[1])[:, :k], want) and not parts[:, :, k:].any()
+        return
+    # three bf16 parts hold 24 bits and more of the fp32 sum
+    assert ((parts.sum(0) - want).abs() <= want.abs() * 2.0 ** -23).all()
+    assert torch.allclose(c.bcol.cpu().double(), Bd.square().sum(0).sqrt(), rtol=2.0 ** -23, atol=0)
+    frob = torch.stack([Bd[:, lo:lo + block].square().sum().sqrt() for lo in range(0, n, block)])
+    assert torch.allclose(c.bfrob.cpu().double(), frob, rtol=2.0 ** -23, atol=0)
