@@ -113,16 +113,17 @@ __device__ __forceinline__ void pack_signs8(const float* sp, uint32_t* sg2) {
 // The four sums of the (row, block) pair each lane keeps: a wave reads 64 consecutive pairs starting at `base`;
 // lane l ends up with pair base + (l & 3) * 16 + (l >> 2).  Four lanes share a pair in each of four rounds; all
 // sixteen 16-byte loads are issued before any is used (256 bytes per lane in flight).  A block narrower than 128 (a
-// row's last) is read the same way, its columns past the end dropped, with its own width's signs: 577-wide rows, a
-// fifth of whose blocks are 65 wide, take 41 us for 64 MB, from 114 us with element loads for every block of
-// rows that are not 16-byte aligned.  Strided rows, and rows of fewer than 8 columns, take an element-wise path.
-// NARROW: whether narrower blocks are read so (they cost 20 registers, a wave a SIMD: 4096 x 14336 35 and 42 us
-// without and with them, so passes over whole blocks leave them out; blocks_narrow).
+// row's last) is read the same way, its columns past the end dropped, with its own width's signs (ns2, lane_signs_last).
+// Strided rows, and rows of fewer than 8 columns, take an element-wise path.
+// NARROW: whether narrower blocks are read so (they cost registers: 4096 x 14336 35 and 42 us without and with them, so
+// passes over whole blocks leave them out; blocks_narrow).  In a round that holds a narrower block every lane drops and picks
+// its signs (a full block drops nothing); with a path of its own for them such rounds took both, and the signs'
+// loads in turn: 96 x 577 x 577, where most rounds do, 39 us, from 41.
 template <int DT, bool NARROW>
-__device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane, const uint32_t* sg2, float& my_pl,
-                                          float& my_sg, float& my_sq, float& my_ab) {
+__device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane, const uint32_t* sg2,
+                                          const uint32_t* ns2, float& my_pl, float& my_sg, float& my_sq, float& my_ab) {
   const int q = lane & 3;
-  int how[4];                           // 0: elements, 1: a full block, 2: a narrower one
+  int how[4];                           // 0: elements, 1: a full block, 2: a narrower one, 3: a narrower last one
   u32x4 v[4][4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
@@ -139,7 +140,7 @@ __device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[g][j] = load16_any(yr + 8 * (q + 4 * j));
       } else if (NARROW && jb * a.bs + wid >= 8) {
-        how[g] = 2;
+        how[g] = last ? 3 : 2;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int c0 = 8 * (q + 4 * j);
@@ -153,39 +154,43 @@ __device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane
   for (int g = 0; g < 4; ++g) {
     const int64_t p = base + g * 16 + (lane >> 2);
     float pl = 0.f, sg = 0.f, sq = 0.f, ab = 0.f;
-    if (how[g] == 1) {
+    if (NARROW && __builtin_amdgcn_ballot_w64(how[g] >= 2)) {
+      if (how[g]) {
+        const bool last = how[g] == 3;
+        const int wid = last ? (int)a.rem : (int)a.bs;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int sh = 8 * (q + 4 * j) + 8 - wid;
+          uint32_t ns[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ns[e] = last ? ns2[4 * j + e] : sg2[4 * j + e];
+          acc8<DT>(drop_low(v[g][j], sh < 0 ? 0 : sh < 8 ? sh : 8), ns, pl, sg, sq, ab);
+        }
+      }
+    } else if (how[g] == 1) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc8<DT>(v[g][j], &sg2[j * 4], pl, sg, sq, ab);
-    } else if (p < a.npairs) {
+    }
+    if (how[g] == 0 && p < a.npairs) {
       int64_t b, r, jb;
       pair_index(a, p, b, r, jb);
       const bool last = (jb == a.nb - 1) && (a.rem > 0);
       const int wid = (int)(last ? a.rem : a.bs);
       const float* sp = last ? a.s_last : a.s_full;
-      if (NARROW && how[g] == 2) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int c0 = 8 * (q + 4 * j), sh = c0 + 8 - wid;
-          uint32_t ns[4];
-          pack_signs8<DT>(sp + c0, ns);
-          acc8<DT>(sh > 0 ? drop_low(v[g][j], sh < 8 ? sh : 8) : v[g][j], ns, pl, sg, sq, ab);
-        }
-      } else {
-        const uint16_t* yr = a.y + b * a.sb + r * a.sm + jb * a.bs * a.sn;
+      const uint16_t* yr = a.y + b * a.sb + r * a.sm + jb * a.bs * a.sn;
 #pragma unroll 1
-        for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll 1
-          for (int e = 0; e < 8; ++e) {
-            const int c = 8 * (q + 4 * j) + e;
-            if (c < wid) {
-              float x = half_to_f32<DT>(yr[c * a.sn]);
-              pl += x;
-              sg = fmaf(x, sp[c], sg);
-              sq = fmaf(x, x, sq);
-              ab += fabsf(x);
-            }
+        for (int e = 0; e < 8; ++e) {
+          const int c = 8 * (q + 4 * j) + e;
+          if (c < wid) {
+            float x = half_to_f32<DT>(yr[c * a.sn]);
+            pl += x;
+            sg = fmaf(x, sp[c], sg);
+            sq = fmaf(x, x, sq);
+            ab += fabsf(x);
           }
-      }
+        }
     }
     pl = quad_sum(pl); sg = quad_sum(sg); sq = quad_sum(sq); ab = quad_sum(ab);
     if (q == g) { my_pl = pl; my_sg = sg; my_sq = sq; my_ab = ab; }
@@ -198,4 +203,11 @@ template <int DT>
 __device__ __forceinline__ void lane_signs(const YView& a, int q, uint32_t* sg2) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) pack_signs8<DT>(a.s_full + 8 * (q + 4 * j), &sg2[j * 4]);
+}
+
+// The signs of the same columns of the last, narrower block (pair_sums' ns2)
+template <int DT>
+__device__ __forceinline__ void lane_signs_last(const YView& a, int q, uint32_t* ns2) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) pack_signs8<DT>(a.s_last + 8 * (q + 4 * j), &ns2[j * 4]);
 }

@@ -195,6 +195,11 @@ constexpr int SDC_SLOT_FLOATS = SDC_SLOTS * SDC_SLOT_WORDS * 2;          // work
 __device__ __forceinline__ void sdc_raise_worst(int64_t* res, unsigned long long* slots, int64_t key, int64_t keyd,
                                                 int64_t seen0, int64_t seen1) {
   if (key <= seen0 && keyd <= seen1) return;
+  if (!slots) {                                                          // (a pass of few workgroups)
+    if (key > seen0) atomicMax((unsigned long long*)res, (unsigned long long)key);
+    if (keyd > seen1) atomicMax((unsigned long long*)(res + 1), (unsigned long long)keyd);
+    return;
+  }
   const uint32_t xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11));        // HW_REG_XCC_ID, bits 0 .. 3
   unsigned long long* s = slots + SDC_SLOT_WORDS * (xcc % SDC_SLOTS);
   const unsigned long long k0 = (unsigned long long)key, k1 = (unsigned long long)keyd;
@@ -204,12 +209,12 @@ __device__ __forceinline__ void sdc_raise_worst(int64_t* res, unsigned long long
   if (k0 > o0 && key > seen0) atomicMax((unsigned long long*)res, k0);
   if (k1 > o1 && keyd > seen1) atomicMax((unsigned long long*)(res + 1), k1);
 }
-// (called by every thread of one workgroup of an earlier kernel; `sets` sets of slots, null: none)
+// (called by every thread of one workgroup of an earlier kernel, at its end: nothing there waits for the stores; at its
+// start they kept the one workgroup a microsecond behind the others, of 28 us for a whole 1024^3 check; `sets` sets
+// of slots, null: none)
 __device__ __forceinline__ void sdc_clear_slots(unsigned long long* slots, int sets, int t, int threads) {
-  if (slots) {
+  if (slots)
     for (int i = t; i < sets * SDC_SLOTS * SDC_SLOT_WORDS; i += threads) slots[i] = 0ull;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (the GEMMs count their own loads from here on)
-  }
 }
 
 // bits of a float as an int64 holding the unsigned 32-bit pattern

@@ -147,7 +147,6 @@ __global__ __launch_bounds__(NT) void expected_gemm_kernel(GemmArgs g) {
   using T = Tile<WGN, NP>;
   __shared__ __attribute__((aligned(16))) uint16_t lds[NBUF][T::ROWS * KS];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, NT);
   const int wm = w / WGN, wn = w % WGN;
   const int64_t nrt = sdc_cdiv(g.m, T::TM) + (g.goffs ? g.ngroups : 0), nct = sdc_cdiv(g.N, T::TN);
   // XCD-aware order: block b runs on XCD b % 8; give XCD x the x-th eighth of the tiles (column tile fastest)
@@ -446,6 +445,7 @@ __global__ __launch_bounds__(NT) void expected_gemm_kernel(GemmArgs g) {
       }
     }
   }
+  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, NT);
 }
 
 template <int MODE, int WGN>
@@ -535,7 +535,6 @@ __global__ __launch_bounds__(64 * RS_WAVES, 1) void rs_gemm_kernel(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[RS_WAVES * ABUF * RS_SEGB];
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, 64 * RS_WAVES);
   const int r = lane & 31, h = lane >> 5;
   const int64_t N = g.N, m = g.m;
   const int64_t nct = sdc_cdiv(N, TC), ncf = sdc_cdiv(N, 32);
@@ -704,6 +703,7 @@ __global__ __launch_bounds__(64 * RS_WAVES, 1) void rs_gemm_kernel(GemmArgs g) {
       }
     }
   }
+  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, 64 * RS_WAVES);
 }
 
 // ------------------------------------------------------------------------- register-streamed GEMM, tall tiles
@@ -748,7 +748,6 @@ __global__ __launch_bounds__(64 * NW, TRF == 4 ? 1 : 2) void rs_gemm_tall_kernel
   __shared__ float xred[XNORM ? NW : 1][XNORM ? TR : 1][2];
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, 64 * NW);
   const int r = lane & 31, h = lane >> 5;
   const int64_t N = g.N, m = g.m;
   // (tile indices in 32 bits, their divisions by run-time divisors the short unsigned ones: the launcher keeps the
@@ -1160,6 +1159,7 @@ __global__ __launch_bounds__(64 * NW, TRF == 4 ? 1 : 2) void rs_gemm_tall_kernel
       }
     }
   }
+  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, 64 * NW);
 }
 
 #undef SDC_TALL_WAIT_B

@@ -42,7 +42,6 @@ __global__ __launch_bounds__(64 * NW, TCF == 1 ? 2 : 1) void lane_gemm_kernel(Ge
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int r = lane & 31, h = lane >> 5;
-  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, 64 * NW);
   const int64_t m = g.m, k = g.k, N = g.N;
   const uint32_t nct = ((uint32_t)N + TC - 1) / TC, ncf = ((uint32_t)N + 31) / 32;
   const uint32_t tiles = (uint32_t)((m + TR - 1) / TR) * nct;
@@ -339,6 +338,7 @@ __global__ __launch_bounds__(64 * NW, TCF == 1 ? 2 : 1) void lane_gemm_kernel(Ge
       }
     }
   }
+  if (blockIdx.x == 0) sdc_clear_slots(g.slots, g.slot_sets, t, 64 * NW);
 }
 
 template <int DT, int TCF>

@@ -214,13 +214,15 @@ __global__ __launch_bounds__(256) void serve_fused_kernel(ScoreArgs a) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, q = lane & 3;
   uint32_t sg2[16];
   lane_signs<DT>(a.yv, q, sg2);
+  uint32_t ns2[GEN ? 16 : 1];
+  if constexpr (GEN) lane_signs_last<DT>(a.yv, q, ns2);
   LaneBest best;
   const int64_t tiles = (a.npairs + 63) / 64;
   for (int64_t tile = (int64_t)blockIdx.x * 4 + w; tile < tiles; tile += (int64_t)gridDim.x * 4) {
     const int64_t base = tile * 64, p = base + q * 16 + (lane >> 2);
     const PairE<NS> pe = load_pair_e<NS>(a, p);
     float pl, sg, sq, ab;
-    pair_sums<DT, GEN>(a.yv, base, lane, sg2, pl, sg, sq, ab);
+    pair_sums<DT, GEN>(a.yv, base, lane, sg2, ns2, pl, sg, sq, ab);
     score_pair_e<DT, NS, GEN>(a, p, pl, sg, sq, ab, pe, best);
   }
   report_wg<DT>(a, best);
@@ -233,11 +235,13 @@ __global__ __launch_bounds__(256) void serve_sums_kernel(ScoreArgs a, float* __r
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, q = lane & 3;
   uint32_t sg2[16];
   lane_signs<DT>(a.yv, q, sg2);
+  uint32_t ns2[16];
+  lane_signs_last<DT>(a.yv, q, ns2);
   const int64_t tiles = (a.npairs + 63) / 64;
   for (int64_t tile = (int64_t)blockIdx.x * 4 + w; tile < tiles; tile += (int64_t)gridDim.x * 4) {
     const int64_t base = tile * 64;
     float pl, sg, sq, ab;
-    pair_sums<DT, true>(a.yv, base, lane, sg2, pl, sg, sq, ab);
+    pair_sums<DT, true>(a.yv, base, lane, sg2, ns2, pl, sg, sq, ab);
     const int64_t p = base + q * 16 + (lane >> 2);
     if (p < a.npairs) {
       sums[p] = pl;

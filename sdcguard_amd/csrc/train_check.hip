@@ -363,6 +363,7 @@ struct TrainArgs {
   int64_t sbias_b, sbias_m, sbias_n;
   float alpha, beta, u, h, abs_floor, l1c, zt, lim_a, capk;
   int64_t* result;                 // [key, key of the noise, unjudged]
+  unsigned long long* slots;       // one row's result slots, cleared by the GEMM (sdc_raise_worst), or null
   float* zdump;
   const int64_t* goffs;            // grouped rows: cumulative group ends (device), or null
   int64_t ngroups;
@@ -378,35 +379,51 @@ struct PairE {
   float e0, e1, asq, asum;
 };
 
-// (MORE: planes past NS are added too)
-template <int NS = SDC_MAX_SPLITS, bool MORE = true>
-__device__ __forceinline__ PairE pair_expected(const TrainArgs& a, int64_t eb, int64_t r, int64_t jb) {
+// The first NS planes' values, loaded and not yet added
+template <int NS>
+struct PairPlanes {
+  float2 ev[NS];
+  float xa[NS], xb[NS];
+};
+
+template <int NS>
+__device__ __forceinline__ PairPlanes<NS> pair_planes(const TrainArgs& a, int64_t eb, int64_t r, int64_t jb) {
   // E planes row-major ([m][ncols]: plain and signed adjacent) or transposed ([ncols][m]: adjacent rows)
   const float* ep = a.et ? a.E + ((eb * a.splits) * a.ncols + 2 * jb) * a.cv.m + r
                          : a.E + ((eb * a.splits) * a.cv.m + r) * a.ncols + 2 * jb;
   const float* xp = a.XN + (eb * a.splits) * 2 * a.cv.m + r;
   const int64_t estep = a.cv.m * a.ncols, xstep = 2 * a.cv.m;
-  float2 ev[NS];
-  float xa[NS], xb[NS];
+  PairPlanes<NS> pp;
   // loads unconditional, so all are in flight at once (a split index past a.splits reads split 0, not added)
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     const int64_t sc = s < a.splits ? s : 0;
-    if (a.et) ev[s] = make_float2(ep[sc * estep], ep[sc * estep + a.cv.m]);
-    else ev[s] = *reinterpret_cast<const float2*>(ep + sc * estep);
-    xa[s] = xp[sc * xstep];
-    xb[s] = xp[sc * xstep + a.cv.m];
+    if (a.et) pp.ev[s] = make_float2(ep[sc * estep], ep[sc * estep + a.cv.m]);
+    else pp.ev[s] = *reinterpret_cast<const float2*>(ep + sc * estep);
+    pp.xa[s] = xp[sc * xstep];
+    pp.xb[s] = xp[sc * xstep + a.cv.m];
   }
-  PairE pe{ev[0].x, ev[0].y, xa[0], xb[0]};
+  return pp;
+}
+
+// (MORE: planes past NS are loaded and added too)
+template <int NS, bool MORE>
+__device__ __forceinline__ PairE add_planes(const TrainArgs& a, int64_t eb, int64_t r, int64_t jb,
+                                            const PairPlanes<NS>& pp) {
+  PairE pe{pp.ev[0].x, pp.ev[0].y, pp.xa[0], pp.xb[0]};
 #pragma unroll
   for (int s = 1; s < NS; ++s)
     if (s < a.splits) {
-      pe.e0 += ev[s].x;
-      pe.e1 += ev[s].y;
-      pe.asq += xa[s];
-      pe.asum += xb[s];
+      pe.e0 += pp.ev[s].x;
+      pe.e1 += pp.ev[s].y;
+      pe.asq += pp.xa[s];
+      pe.asum += pp.xb[s];
     }
   if (MORE && a.splits > NS) {                   // (a short GEMM's further planes)
+    const float* ep = a.et ? a.E + ((eb * a.splits) * a.ncols + 2 * jb) * a.cv.m + r
+                           : a.E + ((eb * a.splits) * a.cv.m + r) * a.ncols + 2 * jb;
+    const float* xp = a.XN + (eb * a.splits) * 2 * a.cv.m + r;
+    const int64_t estep = a.cv.m * a.ncols, xstep = 2 * a.cv.m;
 #pragma unroll 8
     for (int64_t s = NS; s < a.splits; ++s) {
       pe.e0 += ep[s * estep];
@@ -416,6 +433,11 @@ __device__ __forceinline__ PairE pair_expected(const TrainArgs& a, int64_t eb, i
     }
   }
   return pe;
+}
+
+template <int NS = SDC_MAX_SPLITS, bool MORE = true>
+__device__ __forceinline__ PairE pair_expected(const TrainArgs& a, int64_t eb, int64_t r, int64_t jb) {
+  return add_planes<NS, MORE>(a, eb, r, jb, pair_planes<NS>(a, eb, r, jb));
 }
 
 // pe: the pair's expected sums when the caller has them (loaded ahead of C), else null
@@ -504,21 +526,31 @@ __device__ __forceinline__ void train_pair(const TrainArgs& a, int64_t p, float 
   best.keyd = k2 > best.keyd ? k2 : best.keyd;
 }
 
-// GEN: C has blocks narrower than 128, or more than SDC_MAX_SPLITS planes
-template <int DT, bool GEN>
+// Each wave walks tiles of 64 pairs with a grid stride; a tile's expected sums (NS planes) are loaded before its outputs,
+// so both arrive in one round trip.  Measured, 4096 x 14336: 33 us (117 MB; 35 us with the sums loaded after the outputs
+// and every workgroup's keys going straight to a row that starts at zero).
+// GEN: C has blocks narrower than 128, or more than NS planes
+template <int DT, int NS, bool GEN>
 __global__ __launch_bounds__(256) void train_score_kernel(TrainArgs a) {
   __shared__ int64_t red_k[4], red_d[4];
   __shared__ int red_u[4];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, q = lane & 3;
   uint32_t sg2[16];
   lane_signs<DT>(a.cv, q, sg2);
+  uint32_t ns2[GEN ? 16 : 1];
+  if constexpr (GEN) lane_signs_last<DT>(a.cv, q, ns2);
   TrainBest best;
   const int64_t tiles = (a.cv.npairs + 63) / 64;
   for (int64_t tile = (int64_t)blockIdx.x * 4 + w; tile < tiles; tile += (int64_t)gridDim.x * 4) {
-    const int64_t base = tile * 64;
+    const int64_t base = tile * 64, p = base + q * 16 + (lane >> 2);
+    int64_t bc, r, jb;
+    pair_index(a.cv, p < a.cv.npairs ? p : a.cv.npairs - 1, bc, r, jb);
+    const int64_t eb = a.e_batched ? bc : 0;
+    const PairPlanes<NS> pp = pair_planes<NS>(a, eb, r, jb);
     float pl, sg, sq, ab;
-    pair_sums<DT, GEN>(a.cv, base, lane, sg2, pl, sg, sq, ab);
-    train_pair<DT, GEN>(a, base + q * 16 + (lane >> 2), pl, sg, sq, ab, best);
+    pair_sums<DT, GEN>(a.cv, base, lane, sg2, ns2, pl, sg, sq, ab);
+    const PairE pe = add_planes<NS, GEN>(a, eb, r, jb, pp);
+    train_pair<DT, GEN>(a, p, pl, sg, sq, ab, best, -1, &pe);
   }
   int64_t key = wave_max_i64_dpp(best.key), keyd = wave_max_i64_dpp(best.keyd);   // (every lane active)
   int unk = wave_sum_i32_dpp(best.unk);
@@ -534,8 +566,7 @@ __global__ __launch_bounds__(256) void train_score_kernel(TrainArgs a) {
     }
     int64_t* res = a.result;
     const int64_t s0 = __atomic_load_n(res, __ATOMIC_RELAXED), s1 = __atomic_load_n(res + 1, __ATOMIC_RELAXED);
-    if (k0 > s0) atomicMax((unsigned long long*)res, (unsigned long long)k0);
-    if (d0 > s1) atomicMax((unsigned long long*)(res + 1), (unsigned long long)d0);
+    sdc_raise_worst(res, a.slots, k0, d0, s0, s1);
     if (un > 0) atomicAdd((unsigned long long*)(res + 2), (unsigned long long)un);
   }
 }
@@ -626,8 +657,7 @@ __global__ __launch_bounds__(256) void train_score_t_kernel(TrainArgs a) {
     }
     int64_t* res = a.result;
     const int64_t s0 = __atomic_load_n(res, __ATOMIC_RELAXED), s1 = __atomic_load_n(res + 1, __ATOMIC_RELAXED);
-    if (k0 > s0) atomicMax((unsigned long long*)res, (unsigned long long)k0);
-    if (d0 > s1) atomicMax((unsigned long long*)(res + 1), (unsigned long long)d0);
+    sdc_raise_worst(res, a.slots, k0, d0, s0, s1);
     if (un > 0) atomicAdd((unsigned long long*)(res + 2), (unsigned long long)un);
   }
 }
@@ -676,6 +706,8 @@ __global__ __launch_bounds__(256) void grouped_score_kernel(TrainArgs a) {
   }
   uint32_t sg2[16];
   lane_signs<DT>(a.cv, q, sg2);
+  uint32_t ns2[NARROW ? 16 : 1];
+  if constexpr (NARROW) lane_signs_last<DT>(a.cv, q, ns2);
   __syncthreads();
   const int64_t* offs = gl ? offs_s : a.goffs;
   const int64_t tiles = (a.cv.npairs + 63) / 64;
@@ -692,7 +724,7 @@ __global__ __launch_bounds__(256) void grouped_score_kernel(TrainArgs a) {
     pair_index(a.cv, pc, bc, r, jb);
     const PairE pe = pair_expected<NS, false>(a, 0, r, jb);
     float pl, sg, sq, ab;
-    pair_sums<DT, NARROW>(a.cv, base, lane, sg2, pl, sg, sq, ab);
+    pair_sums<DT, NARROW>(a.cv, base, lane, sg2, ns2, pl, sg, sq, ab);
     grp = group_of(offs, a.ngroups, r);
     if (grp >= 0) train_pair<DT>(a, p, pl, sg, sq, ab, tb, grp, &pe);
     const int64_t last = base + 63 < a.cv.npairs ? base + 63 : a.cv.npairs - 1;
@@ -738,7 +770,7 @@ struct Layout {
   int64_t esplits;                 // E and XN planes the workspace holds (the most any of its GEMMs writes)
   int64_t fragb;                   // bytes of one group's parts in fragment order (grouped: a depth of whole 512s;
                                    //   else one batch, its depth rounded up to 64), or 0
-  int64_t off_b2t, off_part, off_col, off_bmax, off_bias, off_parts, off_frag, off_e, off_xn, total;
+  int64_t off_b2t, off_part, off_col, off_bmax, off_bias, off_parts, off_frag, off_e, off_xn, off_slots, total;
 };
 
 // The grouped check's expected side runs on the tall-tile GEMM where the depth allows it, over one depth part (the
@@ -776,6 +808,7 @@ Layout layout(int64_t batch_a, int64_t batch_b, int64_t m, int64_t k, int64_t n,
                                                                             sdc_tall_plan(m, k64, L.ncols, false).splits));
   L.off_e = o; o += al(L.nbt * L.esplits * m * L.ncols);
   L.off_xn = o; o += al(L.nbt * L.esplits * 2 * m);
+  L.off_slots = o; o += SDC_SLOT_FLOATS;
   L.total = o;
   return L;
 }
@@ -873,8 +906,8 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
                const void* C, int64_t scb, int64_t scm, int64_t scn, int64_t batch_c, int64_t m, int64_t k, int64_t bs,
                const Layout& L, const BConsts& bc, const void* bias, int bias_kind, int64_t sbias_b, int64_t sbias_m,
                int64_t sbias_n, float alpha, float beta, float z, float abs_floor, const float* s_full,
-               const float* s_last, int64_t* result, float* E, float* XN, float* scores_out, const int64_t* goffs,
-               hipStream_t stream);
+               const float* s_last, int64_t* result, float* E, float* XN, unsigned long long* slots, float* scores_out,
+               const int64_t* goffs, hipStream_t stream);
 
 // The check of sdc_matmul_check, or (goffs set) of sdc_grouped_check: batch_b groups of B over one tall A / C.
 int run_check(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, int64_t batch_a, const void* B,
@@ -902,7 +935,7 @@ int run_check(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, i
   if (rc != SDC_OK) return rc;
   return check_with(dtype, A, sab, sam, sak, batch_a, batch_b, C, scb, scm, scn, batch_c, m, k, bs, L, bc, bias,
                     bias_kind, sbias_b, sbias_m, sbias_n, alpha, beta, z, abs_floor, s_full, s_last, result,
-                    ws + L.off_e, ws + L.off_xn, scores_out, goffs, stream);
+                    ws + L.off_e, ws + L.off_xn, (unsigned long long*)(ws + L.off_slots), scores_out, goffs, stream);
 }
 
 // The expected-side GEMM and the scoring pass of a check whose B-side constants are made (bc).
@@ -910,8 +943,8 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
                const void* C, int64_t scb, int64_t scm, int64_t scn, int64_t batch_c, int64_t m, int64_t k, int64_t bs,
                const Layout& L, const BConsts& bc, const void* bias, int bias_kind, int64_t sbias_b, int64_t sbias_m,
                int64_t sbias_n, float alpha, float beta, float z, float abs_floor, const float* s_full,
-               const float* s_last, int64_t* result, float* E, float* XN, float* scores_out, const int64_t* goffs,
-               hipStream_t stream) {
+               const float* s_last, int64_t* result, float* E, float* XN, unsigned long long* slots, float* scores_out,
+               const int64_t* goffs, hipStream_t stream) {
   const bool grouped = goffs != nullptr;
   const int64_t nbt = grouped ? 1 : (batch_a > batch_b ? batch_a : batch_b);
   GemmArgs g{};
@@ -919,6 +952,7 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
   g.B = bc.parts; g.sbb = batch_b > 1 ? 3 * L.ncols * L.kp : 0; g.sbc = L.kp;
   g.m = m; g.k = k; g.N = L.ncols; g.splits = L.splits;
   g.E = E; g.XN = XN;
+  g.slots = grouped ? nullptr : slots; g.slot_sets = 1;         // (grouped: a result row per group, few workgroups each)
   const bool c_t = !grouped && scm == 1 && scn != 1 && L.nb < 65536 && batch_c < 65536;   // C read down columns
   g.et = c_t;
   g.prof_name = "train_gemm";
@@ -980,7 +1014,7 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
   ta.zt = z;
   ta.lim_a = dtype == SDC_BF16 ? 1e18f : 65504.f;
   ta.capk = (float)(1.02 + (double)k * 2.384185791015625e-07);
-  ta.result = result; ta.zdump = scores_out;
+  ta.result = result; ta.slots = g.slots; ta.zdump = scores_out;
   ta.goffs = goffs; ta.ngroups = grouped ? batch_b : 0;
   SdcProf prof("train_score", stream);
   ta.et = e_t;
@@ -1012,11 +1046,18 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
     const int64_t tiles = sdc_cdiv(ta.cv.npairs, 64);
     const unsigned grid = (unsigned)(sdc_cdiv(tiles, 4) < 1024 ? sdc_cdiv(tiles, 4) : 1024);
     const bool gen = blocks_narrow(ta.cv) || ta.splits > SDC_MAX_SPLITS;
+    // a slot's maxima take about 1.8 us before the row's, the row's own about 28 ns a workgroup: slots from 64
+    // workgroups up (32 of them, 1024^3: 28.8 us a check with slots, 27.9 without; 1024, 4096 x 14336: 33 and 35 us)
+    if (grid < 64) ta.slots = nullptr;
     const dim3 g1(grid), b1(256);
-    if (dtype == SDC_BF16 && gen) hipLaunchKernelGGL((train_score_kernel<SDC_BF16, true>), g1, b1, 0, stream, ta);
-    else if (dtype == SDC_BF16) hipLaunchKernelGGL((train_score_kernel<SDC_BF16, false>), g1, b1, 0, stream, ta);
-    else if (gen) hipLaunchKernelGGL((train_score_kernel<SDC_FP16, true>), g1, b1, 0, stream, ta);
-    else hipLaunchKernelGGL((train_score_kernel<SDC_FP16, false>), g1, b1, 0, stream, ta);
+    auto go = [&](auto dt) {
+      constexpr int DT = decltype(dt)::value;
+      if (gen) hipLaunchKernelGGL((train_score_kernel<DT, SDC_MAX_SPLITS, true>), g1, b1, 0, stream, ta);
+      else if (ta.splits <= 2) hipLaunchKernelGGL((train_score_kernel<DT, 2, false>), g1, b1, 0, stream, ta);
+      else hipLaunchKernelGGL((train_score_kernel<DT, SDC_MAX_SPLITS, false>), g1, b1, 0, stream, ta);
+    };
+    if (dtype == SDC_BF16) go(std::integral_constant<int, SDC_BF16>{});
+    else go(std::integral_constant<int, SDC_FP16>{});
   }
   SDC_LAUNCH_CHECK();
   return SDC_OK;
@@ -1143,7 +1184,7 @@ extern "C" int sdc_grouped_check_consts(int dtype, const void* A, int64_t sam, i
   // (the bias's block sums are part of the constants; has_bias says whether the layer has one)
   return check_with(dtype, A, 0, sam, sak, 1, groups, C, 0, scm, scn, 1, rows, k, bs, L, bc, nullptr, has_bias ? 1 : 0,
                     0, 0, 0, 1.f, 1.f, z, abs_floor, s_full, s_last, results, ws, ws + (L.off_xn - L.off_e),
-                    scores_out, offs, stream);
+                    nullptr, scores_out, offs, stream);
 }
 
 extern "C" int sdc_grouped_check(int dtype, const void* A, int64_t sam, int64_t sak, const void* B, int64_t sbg,
