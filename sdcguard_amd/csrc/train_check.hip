@@ -1044,15 +1044,20 @@ int check_with(int dtype, const void* A, int64_t sab, int64_t sam, int64_t sak, 
     else hipLaunchKernelGGL(train_score_t_kernel<SDC_FP16>, grid, dim3(256), 0, stream, ta);
   } else {
     const int64_t tiles = sdc_cdiv(ta.cv.npairs, 64);
-    const unsigned grid = (unsigned)(sdc_cdiv(tiles, 4) < 1024 ? sdc_cdiv(tiles, 4) : 1024);
     const bool gen = blocks_narrow(ta.cv) || ta.splits > SDC_MAX_SPLITS;
+    // the workgroups that fit the chip at once: three a CU, two where narrower blocks take registers (four a CU: the
+    // fourth waits for a place and ends alone; 1024 x 50257 with its two products 247 and 242 us, 96 x 577 x 577 62
+    // and 60 us)
+    const int64_t most = gen ? 512 : 768;
+    const unsigned grid = (unsigned)(sdc_cdiv(tiles, 4) < most ? sdc_cdiv(tiles, 4) : most);
     // a slot's maxima take about 1.8 us before the row's, the row's own about 28 ns a workgroup: slots from 64
     // workgroups up (32 of them, 1024^3: 28.8 us a check with slots, 27.9 without; 1024, 4096 x 14336: 33 and 35 us)
     if (grid < 64) ta.slots = nullptr;
     const dim3 g1(grid), b1(256);
     auto go = [&](auto dt) {
       constexpr int DT = decltype(dt)::value;
-      if (gen) hipLaunchKernelGGL((train_score_kernel<DT, SDC_MAX_SPLITS, true>), g1, b1, 0, stream, ta);
+      if (gen && ta.splits <= 2) hipLaunchKernelGGL((train_score_kernel<DT, 2, true>), g1, b1, 0, stream, ta);
+      else if (gen) hipLaunchKernelGGL((train_score_kernel<DT, SDC_MAX_SPLITS, true>), g1, b1, 0, stream, ta);
       else if (ta.splits <= 2) hipLaunchKernelGGL((train_score_kernel<DT, 2, false>), g1, b1, 0, stream, ta);
       else hipLaunchKernelGGL((train_score_kernel<DT, SDC_MAX_SPLITS, false>), g1, b1, 0, stream, ta);
     };
