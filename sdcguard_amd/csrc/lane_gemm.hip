@@ -32,6 +32,31 @@ enum { DEPTH = 0, ROWS = 1 };
 typedef u32x2 __attribute__((aligned(2))) u32x2_any;        // 8 and 16 bytes at any 2-byte address
 typedef u32x4 __attribute__((aligned(2))) u32x4_lane;
 
+// Which element of a 128 x 32 TCF tile lane l of wave w stores at step s of the row-major epilogue: columns col .. + 3 of
+// row `row`.  Every column it reads from LDS has to be one of the tile's own: the waves' sums are a tile after the other
+// there, and nothing follows the last.
+template <int TCF>
+struct RowMajor {
+  static constexpr int TC = 32 * TCF, LANES = TC / 4, ROWS_PER = 64 / LANES, STEPS = TR / (ROWS_PER * NW);
+  static constexpr int col(int l) { return 4 * (l % LANES); }
+  static constexpr int row(int w, int s, int l) { return w * (TR / NW) + ROWS_PER * s + l / LANES; }
+  // every element of the tile once, none outside it
+  static constexpr bool covers_tile() {
+    bool seen[TR * TC / 4] = {};
+    for (int w = 0; w < NW; ++w)
+      for (int s = 0; s < STEPS; ++s)
+        for (int l = 0; l < 64; ++l) {
+          const int r = row(w, s, l), c = col(l);
+          if (r < 0 || r >= TR || c < 0 || c + 4 > TC || seen[(r * TC + c) / 4]) return false;
+          seen[(r * TC + c) / 4] = true;
+        }
+    for (bool b : seen)
+      if (!b) return false;
+    return true;
+  }
+};
+static_assert(RowMajor<1>::covers_tile() && RowMajor<2>::covers_tile(), "the row-major epilogue stays in the tile's sums");
+
 // MODE: ROWS needs g.sam 1, g.sak >= g.m >= 4; DEPTH needs g.sak 1.  TCF: 32-column fragments of the tile
 template <int DT, int MODE, int TCF>
 __global__ __launch_bounds__(64 * NW, TCF == 1 ? 2 : 1) void lane_gemm_kernel(GemmArgs g) {
@@ -312,11 +337,12 @@ __global__ __launch_bounds__(64 * NW, TCF == 1 ? 2 : 1) void lane_gemm_kernel(Ge
       }
     }
   } else {
-    // row-major plane [m][N]: an instruction writes 4 rows x 64 columns
-    const int c4 = 4 * (lane & 15);
+    // row-major plane [m][N]: an instruction writes whole rows of the tile, lane l four columns of one (RowMajor)
+    using Map = RowMajor<TCF>;
+    const int c4 = Map::col(lane);
 #pragma unroll
-    for (int gq = 0; gq < TR / (4 * NW); ++gq) {
-      const int rl = w * (TR / NW) + 4 * gq + (lane >> 4);
+    for (int gq = 0; gq < Map::STEPS; ++gq) {
+      const int rl = Map::row(w, gq, lane);
       f32x4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
