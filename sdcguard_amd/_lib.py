@@ -10,6 +10,7 @@ import os
 import threading
 
 import torch
+from torch.utils.weak import WeakIdKeyDictionary
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsdcguard_hip.so")
@@ -136,6 +137,81 @@ def _raw_stream(device: torch.device) -> int:
 def stream_of(t: torch.Tensor) -> int:
     """The raw hipStream_t of the current stream of t's device."""
     return _raw_stream(t.device)
+
+
+def version_of(t: torch.Tensor):
+    """t's version counter; None for an inference tensor, which has none."""
+    try:
+        return t._version
+    except RuntimeError:
+        return None
+
+
+# How a tensor kept on constants made elsewhere was made: the event behind its kernels (None once it has passed), and the
+# streams ordered behind it.
+class _Made:
+    __slots__ = ("event", "streams")
+
+    def __init__(self, event, stream):
+        self.event, self.streams = event, {stream}
+
+
+_MADE = WeakIdKeyDictionary()
+
+
+def keep(owner: torch.Tensor, name: str, key, out: torch.Tensor) -> torch.Tensor:
+    """Keep `out` on the constants it was made with, on their stream: whatever orders another stream behind the
+    constants orders it behind `out` too."""
+    setattr(owner, name, (key, out, -1))
+    return out
+
+
+def made_with(owner: torch.Tensor, name: str, key):
+    """What `keep` kept on `owner`; None if there is nothing, or it was made from something else."""
+    hit = getattr(owner, name, None)
+    return hit[1] if hit is not None and hit[2] == -1 and hit[0] == key else None
+
+
+def kept(owner: torch.Tensor, name: str, key, stream: int, make) -> torch.Tensor:
+    """The tensor make() queues on `stream` (the device's current one), kept on the tensor `owner` that it is made from and
+    made again when `key` changes.  A later call on another stream first waits for it there (an event, no host wait).
+    While the stream is being captured nothing new is kept (a replay, not the capture, would write it), and a tensor
+    that is not known to be finished is made again within the graph (a captured stream cannot wait for outside work)."""
+    hit = getattr(owner, name, None)
+    if hit is not None and hit[0] == key:
+        return hit[1] if hit[2] == stream or _ready(hit[1], stream) else make()
+    out = make()
+    with torch.cuda.device(out.device):
+        if torch.cuda.is_current_stream_capturing():
+            return out
+        event = torch.cuda.Event()
+        event.record()
+    _MADE[out] = _Made(event, stream)
+    try:
+        setattr(owner, name, (key, out, stream))
+    except (AttributeError, RuntimeError):
+        pass
+    return out
+
+
+def _ready(out: torch.Tensor, stream: int) -> bool:
+    made = _MADE.get(out)
+    if made is None:
+        return False
+    if stream in made.streams:
+        return True
+    with torch.cuda.device(out.device):
+        if torch.cuda.is_current_stream_capturing():
+            if made.event is not None:
+                return False
+        elif made.event is not None:
+            if made.event.query():
+                made.event = None
+            else:
+                made.event.wait()
+        out.record_stream(torch.cuda.current_stream())
+    made.streams.add(stream)
+    return True
 
 
 def require_gpu(*ts) -> None:

@@ -15,7 +15,7 @@ import torch
 
 from . import _lib
 from .checksum import ABS_FLOOR, CheckResult, CheckStat, resolve, sign_table
-from .serve import STATE_COLS, LayerChecksums, _kmajor_parts, _packed_consts, decode
+from .serve import STATE_COLS, LayerChecksums, _fragments, _kmajor_parts, _packed_consts, decode
 
 BLOCK = 128
 
@@ -75,27 +75,6 @@ def check_linear_both(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torc
         return state, row_result
     _lib.check(rc, "sdc_linear_check")
     return state, row_result
-
-
-def _fragments(P: torch.Tensor, ncols: int, k: int) -> Optional[torch.Tensor]:
-    """The layer's parts in the register-streamed GEMM's fragment order (sdc_parts_fragments), made once and kept on
-    the parts tensor (so they live as long as the constants they copy); None where that GEMM does not apply (depth
-    not a multiple of 64, part columns not 16-byte aligned)."""
-    if k % 64 or P.stride(1) % 8 or P.data_ptr() % 16:
-        return None
-    key = (P.data_ptr(), P._version, ncols, k)
-    hit = getattr(P, "_sdc_frag", None)
-    if hit is not None and hit[0] == key:
-        return hit[1]
-    L = _lib.lib()
-    out = torch.empty(int(L.sdc_parts_fragments_bytes(ncols, k)) // 2, dtype=torch.int16, device=P.device)
-    _lib.check(L.sdc_parts_fragments(P.data_ptr(), P.stride(1), ncols, k, out.data_ptr(), _lib.stream_of(P)),
-               "sdc_parts_fragments")
-    try:
-        P._sdc_frag = (key, out)
-    except (AttributeError, RuntimeError):
-        pass
-    return out
 
 
 def _separately(x2, weight, bias, y2, cs, z, abs_floor, state, row_result, col_scores, row_scores) -> None:

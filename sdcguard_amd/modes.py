@@ -62,6 +62,13 @@ class QuantChecksums:
 
     @classmethod
     def make(cls, B: torch.Tensor, sb: Optional[torch.Tensor] = None, block: int = BLOCK) -> "QuantChecksums":
+        consts = cls._make(B, sb, block)
+        if consts.parts.is_cuda:
+            _fragments(consts.kind, consts.parts, consts.parts.shape[1], consts.k, at_make=True)
+        return consts
+
+    @classmethod
+    def _make(cls, B: torch.Tensor, sb: Optional[torch.Tensor], block: int) -> "QuantChecksums":
         if B.dim() != 2:
             raise ValueError("B must be (k, n)")
         k, n = B.shape
@@ -137,34 +144,27 @@ class QuantStat:
     scores: Optional[torch.Tensor] = None
 
 
-def _fp8_fragments(P: torch.Tensor, ncols: int, k: int) -> Optional[torch.Tensor]:
-    """The fp8 weight's parts in the register-streamed GEMM's fragment order, made once and kept on the parts tensor
-    (the GEMM whose tiles fill the GPU reads them; None where it cannot: depth not a multiple of 1024)."""
-    if k % 1024 or P.stride(1) % 8 or P.data_ptr() % 16:
-        return None
-    from .linear import _fragments
-    return _fragments(P, ncols, k)
-
-
-def _i8_fragments(P: torch.Tensor, ncols: int, k: int) -> Optional[torch.Tensor]:
-    """The int8 weight's two digit planes in the tall-tile GEMM's int8 fragment order (sdc_digit_fragments), made
-    once and kept on the parts tensor; None where that GEMM does not apply (depth not a multiple of 1024)."""
+def _fragments(kind: str, P: torch.Tensor, ncols: int, k: int, at_make: bool = False) -> Optional[torch.Tensor]:
+    """The weight's parts (fp8) or two digit planes (int8, sdc_digit_fragments) in the tall-tile GEMM's fragment order,
+    kept on the parts tensor: made with it by QuantChecksums.make (at_make), at the first check for constants made
+    elsewhere.  None where that GEMM does not apply: depth not a multiple of 1024."""
     from . import _lib
     if k % 1024 or P.stride(1) % 8 or P.data_ptr() % 16:
         return None
-    key = (P.data_ptr(), P._version, ncols, k)
-    hit = getattr(P, "_sdc_frag8", None)
-    if hit is not None and hit[0] == key:
-        return hit[1]
-    L = _lib.lib()
-    out = torch.empty(int(L.sdc_digit_fragments_bytes(ncols, k)), dtype=torch.uint8, device=P.device)
-    _lib.check(L.sdc_digit_fragments(P.data_ptr(), P.stride(1), ncols, k, out.data_ptr(), _lib.stream_of(P)),
-               "sdc_digit_fragments")
-    try:
-        P._sdc_frag8 = (key, out)
-    except (AttributeError, RuntimeError):
-        pass
-    return out
+    if kind == "fp8":
+        from .serve import _fragments as parts_fragments
+        return parts_fragments(P, ncols, k, at_make)
+    key = (P.data_ptr(), _lib.version_of(P), ncols, k)
+    hit = _lib.made_with(P, "_sdc_digits", key)
+    if hit is not None or (key[1] is None and not at_make):      # (no version: a change would go unnoticed)
+        return hit
+    L, s = _lib.lib(), _lib.stream_of(P)
+
+    def make():
+        out = torch.empty(int(L.sdc_digit_fragments_bytes(ncols, k)), dtype=torch.uint8, device=P.device)
+        _lib.check(L.sdc_digit_fragments(P.data_ptr(), P.stride(1), ncols, k, out.data_ptr(), s), "sdc_digit_fragments")
+        return out
+    return _lib.keep(P, "_sdc_digits", key, make()) if at_make else _lib.kept(P, "_sdc_digits", key, s, make)
 
 
 def quant_zscores(A: torch.Tensor, consts: QuantChecksums, C: torch.Tensor, *, sa: Optional[torch.Tensor] = None,
@@ -196,7 +196,7 @@ def quant_zscores(A: torch.Tensor, consts: QuantChecksums, C: torch.Tensor, *, s
     tab = sign_table(C.device)
     P = consts.parts
     Av = A.view(torch.uint8) if kind == 1 else A
-    frag = _fp8_fragments(P, 2 * nb, k) if kind == 1 else _i8_fragments(P, 2 * nb, k)
+    frag = _fragments(consts.kind, P, 2 * nb, k)
     rc = L.sdc_quant_check(
         kind, Av.data_ptr(), Av.stride(0), P.data_ptr(), P.stride(1), None if frag is None else frag.data_ptr(),
         None if sa is None else sa.data_ptr(),

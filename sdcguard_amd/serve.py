@@ -128,9 +128,10 @@ class LayerChecksums:
         self.pair_rem = _pattern_pair(self.rem, dt, dev) if self.rem else self.pair_full
         self.fingerprint = fingerprint(W)
         # the scoring pass reads one (nb, 12) table per variant: hand the built ones to _packed_consts
-        self.bsum._sdc_packed = (table[0], (self.scale.data_ptr(), self.bmax_bias.data_ptr(), self.b2n.data_ptr()))
-        self._nobias[1]._sdc_packed = (table[1], (self.scale.data_ptr(), self._nobias[0].data_ptr(),
-                                                  self.b2n.data_ptr()))
+        for bmb, bsum, tab in ((self.bmax_bias, self.bsum, table[0]), (*self._nobias, table[1])):
+            _lib.keep(bsum, "_sdc_table", (self.scale.data_ptr(), bmb.data_ptr(), self.b2n.data_ptr()), tab)
+        # and the parts in the tall-tile GEMM's order
+        _fragments(self.parts, 2 * nb, k, at_make=True)
         for t in self.tensors(True) + self._nobias:
             _pin_address(t)
 
@@ -164,21 +165,35 @@ def _kmajor_parts(parts: torch.Tensor, scale: torch.Tensor, nb: int, dt: torch.d
     fp32_sums = parts.shape[1] == 2 * nb
     key = (parts._version, tuple(parts.shape), parts.dtype, dt,
            (scale.data_ptr(), scale._version) if fp32_sums else None)
-    hit = getattr(parts, "_sdc_kmajor", None)
-    if hit is not None and hit[0] == key:
-        return hit[1]
-    with torch.no_grad():
-        if parts.shape[1] == 6 * nb and parts.dtype == dt:
-            out = parts.t().contiguous().t()
-        elif fp32_sums:                                      # plain fp32 B2: split it (scale applies to E after)
-            out = _split3_kmajor(parts.float() / scale.reshape(1, 2 * nb), dt)
-        else:
+
+    def make():
+        with torch.no_grad():
+            if parts.shape[1] == 6 * nb and parts.dtype == dt:
+                return parts.t().contiguous().t()
+            if fp32_sums:                                    # plain fp32 B2: split it (scale applies to E after)
+                return _split3_kmajor(parts.float() / scale.reshape(1, 2 * nb), dt)
             raise ValueError(f"parts of shape {tuple(parts.shape)} don't fit {nb} blocks")
-    try:
-        parts._sdc_kmajor = (key, out)
-    except (AttributeError, RuntimeError):
-        pass
-    return out
+    return _lib.kept(parts, "_sdc_by_column", key, _lib.stream_of(parts), make)
+
+
+def _fragments(P: torch.Tensor, ncols: int, k: int, at_make: bool = False) -> Optional[torch.Tensor]:
+    """The layer's parts in the register-streamed GEMM's fragment order (sdc_parts_fragments), kept on the parts tensor
+    (so they live as long as the constants they copy): made with them by LayerChecksums and QuantChecksums
+    (at_make), at the first check for parts made elsewhere.  None where that GEMM does not apply (depth not a
+    multiple of 64, part columns not 16-byte aligned)."""
+    key = (P.data_ptr(), _lib.version_of(P), ncols, k)
+    hit = _lib.made_with(P, "_sdc_fragments", key)
+    if hit is not None:
+        return hit
+    if k % 64 or P.stride(1) % 8 or P.data_ptr() % 16 or (key[1] is None and not at_make):
+        return None                                          # (no version: a change of the parts would go unnoticed)
+    L, s = _lib.lib(), _lib.stream_of(P)
+
+    def make():
+        out = torch.empty(int(L.sdc_parts_fragments_bytes(ncols, k)) // 2, dtype=torch.int16, device=P.device)
+        _lib.check(L.sdc_parts_fragments(P.data_ptr(), P.stride(1), ncols, k, out.data_ptr(), s), "sdc_parts_fragments")
+        return out
+    return _lib.keep(P, "_sdc_fragments", key, make()) if at_make else _lib.kept(P, "_sdc_fragments", key, s, make)
 
 
 def check_static_impl(x2: torch.Tensor, y2: torch.Tensor, parts: torch.Tensor, pair_full: torch.Tensor,
@@ -218,7 +233,6 @@ def check_static_impl(x2: torch.Tensor, y2: torch.Tensor, parts: torch.Tensor, p
     # the parts in fragment order for the tall-tile GEMM (made once, kept on the parts tensor), where it applies
     frag = None
     if k % 64 == 0 and x2.stride(1) == 1 and x2.data_ptr() % 16 == 0 and (x2.stride(0) * x2.element_size()) % 16 == 0:
-        from .linear import _fragments
         frag = _fragments(P, 2 * nb, k)
     ws_bytes = int(L.sdc_check_static_workspace(m, k, n, bs))
     ws = _lib.workspace(y2.device, ws_bytes)
@@ -240,18 +254,17 @@ def _packed_consts(scale, b2n, b2max, bmax, bmax_bias, bsum) -> torch.Tensor:
     """The per-block constants as one (nb, 12) fp32 table (three 16-byte loads per block in the kernel):
     [scale, bsum, b2n, b2max, bmax, bmax_bias, 0, 0].  Kept on the bsum tensor object (with and without the
     bias, LayerChecksums hands different bsum tensors), so it lives exactly as long as the constants it packs."""
-    packed = getattr(bsum, "_sdc_packed", None)
-    if packed is not None and packed[1] == (scale.data_ptr(), bmax_bias.data_ptr(), b2n.data_ptr()):
-        return packed[0]
-    nb = b2n.shape[0]
-    z = torch.zeros(nb, 2, dtype=torch.float32, device=bsum.device)
-    t = torch.cat([scale.view(nb, 2), bsum.view(nb, 2), b2n.view(nb, 2), b2max.view(nb, 2),
-                   torch.stack([bmax.view(nb), bmax_bias.view(nb)], 1), z], dim=1).contiguous()
-    try:
-        bsum._sdc_packed = (t, (scale.data_ptr(), bmax_bias.data_ptr(), b2n.data_ptr()))
-    except (AttributeError, RuntimeError):
-        pass
-    return t
+    key = (scale.data_ptr(), bmax_bias.data_ptr(), b2n.data_ptr())
+    packed = _lib.made_with(bsum, "_sdc_table", key)
+    if packed is not None:
+        return packed
+
+    def make():
+        nb = b2n.shape[0]
+        z = torch.zeros(nb, 2, dtype=torch.float32, device=bsum.device)
+        return torch.cat([scale.view(nb, 2), bsum.view(nb, 2), b2n.view(nb, 2), b2max.view(nb, 2),
+                          torch.stack([bmax.view(nb), bmax_bias.view(nb)], 1), z], dim=1).contiguous()
+    return _lib.kept(bsum, "_sdc_table", key, _lib.stream_of(bsum), make)
 
 
 def kernel_mode() -> int:
