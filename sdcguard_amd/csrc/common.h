@@ -179,6 +179,14 @@ __device__ __forceinline__ int64_t wave_max_i64_dpp(int64_t v) {
   return r;
 }
 
+// Between a wave's LDS stores and another lane's loads of them (and between loads and the stores that follow), where the wave
+// is the only one at that memory.  A wave's LDS accesses are done in order, so no instruction comes of it, but without it
+// the compiler, which orders one lane's accesses only, may move them past each other.
+__device__ __forceinline__ void sdc_wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // The worst keys of a check's result row (res[0]: key, res[1]: key with its noise; both hold the score's bits in
 // their high half), raised by one thread of a workgroup.  Device-scope maxima on one address from every XCD
 // serialize at about 14 ns each: on a row that starts at zero, as every queued check's does, two for each of a

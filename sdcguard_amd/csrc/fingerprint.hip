@@ -538,12 +538,14 @@ __device__ __forceinline__ void kvm_chunks(const KvArgs& a, const int64_t* rowbl
   };
   const int wslot = (lane & 7) ^ (lane >> 3);                  // load i's piece lane % 8 of row 8 i + lane / 8
   auto process = [&](const u32x4* d, const i32x4* tf) {
+    sdc_wave_lds_fence();
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       // 2-byte words: the low bytes' top bits flipped (lo - 128); 1-byte words as they are
       const u32x4 x = WB == 2 ? d[i] ^ u32x4{0x00800080u, 0x00800080u, 0x00800080u, 0x00800080u} : d[i];
       *reinterpret_cast<u32x4*>(L + (8 * i + (lane >> 3)) * 128 + 16 * wslot) = x;
     }
+    sdc_wave_lds_fence();
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll

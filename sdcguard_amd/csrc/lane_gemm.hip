@@ -159,9 +159,11 @@ __global__ __launch_bounds__(64 * NW, TCF == 1 ? 2 : 1) void lane_gemm_kernel(Ge
     }
   };
   auto store_seg = [&]() {
+    sdc_wave_lds_fence();
 #pragma unroll
     for (int I = 0; I < NAP; ++I)
       *reinterpret_cast<u32x4*>(L + (8 * I + (lane >> 3)) * 128 + 16 * ((lane & 7) ^ (lane >> 3))) = as[I];
+    sdc_wave_lds_fence();
   };
   auto load_b = [&](int j, int sg) {
     const uint16_t* p = bq + (4 * (int64_t)sg + j) * bstep;
@@ -242,8 +244,7 @@ __global__ __launch_bounds__(64 * NW, TCF == 1 ? 2 : 1) void lane_gemm_kernel(Ge
       }
     }
   } else if (seg1 > seg0) {
-    // (the wave's LDS holds one segment: a wave's LDS accesses are done in order, so the next segment's stores follow
-    // this one's reads)
+    // (the wave's LDS holds one segment, stored by some lanes and read by others)
     if (nf > 0) {
       load_seg(0);
 #pragma unroll
