@@ -743,12 +743,13 @@ int acc_run(AccArgs a, const AccLayout& L, uint8_t* ws, hipStream_t stream) {
   a.nb = L.nb; a.nslice = L.nslice; a.nseg = L.nseg; a.nct = L.nct; a.ctg = L.ctg; a.splits = L.splits; a.segs = L.segs;
   a.B2T = (double*)(ws + L.off_b2); a.part = (float*)(ws + L.off_part); a.bstat = (float*)(ws + L.off_bstat);
   a.bsum = (double*)(ws + L.off_bsum); a.bmax = (float*)(ws + L.off_bmax); a.an = (float*)(ws + L.off_an);
-  a.slots = (unsigned long long*)(ws + L.off_slots); a.E = (double*)(ws + L.off_e);
+  a.E = (double*)(ws + L.off_e);
   // 16-byte loads of 8 elements need 8 of them to be there: rows of at least 8 columns, columns of at least 8 depths
   a.bmode = a.sbn == 1 && a.n >= 8 ? BROWS : a.sbk == 1 && a.k >= 8 ? BDEPTH : BELEM;
   a.bwork = L.nslice * L.nb * a.batch_b;
   a.gwork = sdc_cdiv(a.m, 128) * L.ctg * L.splits * a.batch_c;
   const int64_t pgrid = sdc_cdiv(a.batch_c * a.m * L.nb, SPAIRS);
+  a.slots = sdc_slots_for(pgrid, (unsigned long long*)(ws + L.off_slots));
   const int64_t bgrid = a.bwork + sdc_cdiv(a.batch_a * a.m, 4), ggrid = a.gwork + sdc_cdiv(a.batch_b * L.nb + L.nb, 4);
   if (bgrid > 0x7FFFFFFFll || ggrid > 0x7FFFFFFFll) return SDC_EUNSUPPORTED;
   {

@@ -593,7 +593,7 @@ __global__ __launch_bounds__(256) void ypass_kernel(YArgs a) {
     const int64_t d0 = red_d[w0] > red_d[w0 + 1] ? red_d[w0] : red_d[w0 + 1];
     const int un = red_u[w0] + red_u[w0 + 1];
     int64_t* res = t == 0 ? a.state : a.result;
-    sdc_raise_worst(res, a.slots + (t == 0 ? 0 : SDC_SLOTS * SDC_SLOT_WORDS), k0, d0, seen0, seen1);
+    sdc_raise_worst(res, a.slots && t ? a.slots + SDC_SLOTS * SDC_SLOT_WORDS : a.slots, k0, d0, seen0, seen1);
     if (t == 0) {
       if (blockIdx.x == 0 && blockIdx.y == 0) atomicAdd((unsigned long long*)(res + 2), 1ull);
       if (un > 0) atomicAdd((unsigned long long*)(res + 3), (unsigned long long)un);
@@ -702,7 +702,7 @@ int queue_both(const void* x, int64_t sxm, const void* W, int64_t swn, const voi
   gc.m = m; gc.k = k; gc.N = 2 * L.nb; gc.splits = L.scol;
   gc.E = ws + L.off_ecol; gc.XN = nullptr; gc.et = 1;
   gc.prof_name = "col_gemm";
-  gc.slots = (unsigned long long*)(ws + L.off_slots); gc.slot_sets = 2;
+  gc.slots = sdc_slots_for(L.nb * L.mb, (unsigned long long*)(ws + L.off_slots)); gc.slot_sets = 2;
   int rc = SDC_EUNSUPPORTED;
   if (L.rs_col && (parts_frag ||
                    sdc_parts_fragments(parts, spc, 2 * L.nb, k, ws + L.off_fcol, side) == SDC_OK)) {

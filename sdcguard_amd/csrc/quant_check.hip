@@ -670,7 +670,11 @@ extern "C" int sdc_quant_check(int kind, const void* A, int64_t sam, const void*
   g.m = m; g.k = kg; g.N = L.ncols; g.splits = L.splits;
   g.E = ws + L.off_e; g.XN = ws + L.off_xn;
   g.prof_name = kind == 0 ? "quant_gemm_i8" : "quant_gemm_fp8";
-  g.slots = (unsigned long long*)(ws + L.off_slots); g.slot_sets = 1;
+  // result slots only for fp8, whose every wave has a score: an exact int8 check raises the row for wrong blocks alone,
+  // and a few of them wait for a slot longer than for the row (1513 x 1784, eight wrong blocks: 7.6 us with slots, 6.8
+  // without; 2048 x 3968 with one wrong block a row 10.8 and 10.2; 2048 x 4096 wrong in every block 22.2 and 41.4)
+  g.slots = kind == 0 ? nullptr : sdc_slots_for(L.nb * sdc_cdiv(m, 64), (unsigned long long*)(ws + L.off_slots));
+  g.slot_sets = 1;
   int rc = SDC_EUNSUPPORTED;
   int64_t splits = L.splits;
   if (L.tall && tiles && sam % 16 == 0 && (uintptr_t)A % 16 == 0 && spc % 8 == 0 && spc >= k &&

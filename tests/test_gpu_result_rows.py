@@ -20,7 +20,7 @@ def _holds_worst(row, scores):
     assert float(flat[key & 0xFFFFFFFF]) == _z(key)
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 256, 128), (129, 256, 136), (2048, 512, 6144)])
+@pytest.mark.parametrize("m,k,n", [(1, 256, 128), (129, 256, 136), (1152, 128, 896), (1024, 128, 1024), (2048, 512, 6144)])
 def test_linear_rows(m, k, n):
     from sdcguard_amd import LayerChecksums
     from sdcguard_amd.linear import check_linear_both
@@ -45,7 +45,8 @@ def test_linear_rows(m, k, n):
     assert _z(state[0]) > _z(kept[0][0]) and _z(row[0]) > _z(kept[1][0])
 
 
-@pytest.mark.parametrize("mode,m,k,n", [("fp8", 1, 64, 8), ("fp8", 130, 96, 200), ("fp8", 2048, 1024, 6144),
+@pytest.mark.parametrize("mode,m,k,n", [("fp8", 1, 64, 8), ("fp8", 130, 96, 200), ("fp8", 4032, 64, 128),
+                                        ("fp8", 4096, 64, 128), ("fp8", 2048, 1024, 6144),
                                         ("fp8", 2048, 96, 6143), ("int8", 2048, 128, 6144)])
 def test_quant_rows(mode, m, k, n):
     from sdcguard_amd import modes
@@ -70,3 +71,56 @@ def test_quant_rows(mode, m, k, n):
         assert row[2:] == [int((z > 6).sum()), 0]
     if mode == "int8":                                       # the last wrong block's place
         assert row[0] & 0xFFFFFFFF == m * z.shape[1] - 1 and row[2] == 2
+
+
+def _product(m, k, n, la, lc, batch, dt, g):
+    """A, B and C = A @ B (fp32), A and C in a layout: rows or columns contiguous, or rows at odd addresses."""
+    lead = (batch,) if batch else ()
+    a, b = (torch.randn(*lead, *s, device="cuda", generator=g).to(dt) for s in ((m, k), (k, n)))
+    c = a.float() @ b.float()
+
+    def lay(t, how):
+        if how == "cols":
+            return t.transpose(-1, -2).contiguous().transpose(-1, -2)
+        if how == "odd":
+            return torch.cat([t[..., :3], t, t[..., :2]], -1)[..., 3:3 + t.shape[-1]]
+        return t
+    return lay(a, la), b, lambda d: lay(c.to(d), lc)
+
+
+# (each path of the expected side's GEMM before the scores: whole lines, 32- and 64-row tiles, unaligned rows, contiguous
+# columns, neither, batches; below and past 64 scoring workgroups; C by rows, at odd addresses and by columns)
+@pytest.mark.parametrize("m,k,n,la,lc,batch", [
+    (1, 64, 128, "rows", "rows", 0), (32, 64, 64500, "rows", "rows", 0), (60, 128, 35000, "rows", "rows", 0),
+    (2016, 64, 1024, "rows", "rows", 0), (2048, 64, 1024, "rows", "rows", 0), (8192, 64, 1024, "rows", "odd", 0),
+    (2048, 65, 1030, "odd", "rows", 0), (5000, 90, 700, "cols", "rows", 0), (1500, 64, 3000, "rows", "cols", 0),
+    (20000, 100, 300, "cols", "cols", 0), (300, 64, 500, "rows", "rows", 24), (2048, 1000, 1024, "odd", "cols", 0)])
+def test_training_rows(m, k, n, la, lc, batch):
+    from sdcguard_amd import matmul_zscores
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    a, b, c = _product(m, k, n, la, lc, batch, torch.bfloat16, g)
+    c = c(torch.bfloat16)
+    nb = -(-n // 128)
+    z = torch.empty(max(1, batch), m, nb, 2, device="cuda")
+    bad = torch.cat([c[..., :3], c], -1)[..., 3:] if lc == "odd" else c.clone(memory_format=torch.preserve_format)
+    bad[..., m // 2, n // 2] += 1e4
+    for out in (bad, c, bad, c):                             # (a worst call before each clean one: stale slots would hide it)
+        row = matmul_zscores(a, b, out, scores_out=z).result.tolist()
+        _holds_worst(row, z)
+        assert row[2] == 0 and (_z(row[0]) > 6.0) == (out is bad)
+
+
+@pytest.mark.parametrize("m,k,n,lc,batch", [(1, 64, 128, "rows", 0), (1008, 64, 1024, "rows", 0), (1024, 64, 1024, "rows", 0),
+                                            (3000, 65, 1030, "odd", 0), (300, 40, 500, "rows", 24)])
+def test_precise_rows(m, k, n, lc, batch):
+    from sdcguard_amd.checksum import matmul_zscores_acc
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    a, b, c = _product(m, k, n, "rows", lc, batch, torch.bfloat16, g)
+    c = c(torch.float32)
+    z = torch.empty(max(1, batch), m, -(-n // 128), 2, device="cuda")
+    bad = c.clone()
+    bad[..., m // 2, n // 2] += 1e4
+    for out in (bad, c, bad, c):
+        row = matmul_zscores_acc(a, b, out, scores_out=z).result.tolist()
+        _holds_worst(row, z)
+        assert row[2] == 0 and (_z(row[0]) > 6.0) == (out is bad)
