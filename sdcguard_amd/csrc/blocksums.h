@@ -132,19 +132,26 @@ __device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane
     if (p < a.npairs && a.vec) {
       int64_t b, r, jb;
       pair_index(a, p, b, r, jb);
-      const bool last = (jb == a.nb - 1) && (a.rem > 0);
-      const int wid = (int)(last ? a.rem : a.bs);
-      const uint16_t* yr = a.y + b * a.sb + r * a.sm + jb * a.bs;
-      if (wid == 128) {
+      if constexpr (!NARROW) {            // (rows read so hold whole blocks only)
         how[g] = 1;
+        const uint16_t* yr = a.y + b * a.sb + r * a.sm + jb * 128;
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[g][j] = load16_any(yr + 8 * (q + 4 * j));
-      } else if (NARROW && jb * a.bs + wid >= 8) {
-        how[g] = last ? 3 : 2;
+      } else {
+        const bool last = (jb == a.nb - 1) && (a.rem > 0);
+        const int wid = (int)(last ? a.rem : a.bs);
+        const uint16_t* yr = a.y + b * a.sb + r * a.sm + jb * a.bs;
+        if (wid == 128) {
+          how[g] = 1;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int c0 = 8 * (q + 4 * j);
-          v[g][j] = load16_any(yr + (c0 + 8 <= wid ? c0 : wid - 8));
+          for (int j = 0; j < 4; ++j) v[g][j] = load16_any(yr + 8 * (q + 4 * j));
+        } else if (jb * a.bs + wid >= 8) {
+          how[g] = last ? 3 : 2;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int c0 = 8 * (q + 4 * j);
+            v[g][j] = load16_any(yr + (c0 + 8 <= wid ? c0 : wid - 8));
+          }
         }
       }
     }
@@ -154,24 +161,11 @@ __device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane
   for (int g = 0; g < 4; ++g) {
     const int64_t p = base + g * 16 + (lane >> 2);
     float pl = 0.f, sg = 0.f, sq = 0.f, ab = 0.f;
-    if (NARROW && __builtin_amdgcn_ballot_w64(how[g] >= 2)) {
-      if (how[g]) {
-        const bool last = how[g] == 3;
-        const int wid = last ? (int)a.rem : (int)a.bs;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int sh = 8 * (q + 4 * j) + 8 - wid;
-          uint32_t ns[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ns[e] = last ? ns2[4 * j + e] : sg2[4 * j + e];
-          acc8<DT>(drop_low(v[g][j], sh < 0 ? 0 : sh < 8 ? sh : 8), ns, pl, sg, sq, ab);
-        }
-      }
-    } else if (how[g] == 1) {
+    auto whole = [&]() {
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc8<DT>(v[g][j], &sg2[j * 4], pl, sg, sq, ab);
-    }
-    if (how[g] == 0 && p < a.npairs) {
+    };
+    auto elements = [&]() {
       int64_t b, r, jb;
       pair_index(a, p, b, r, jb);
       const bool last = (jb == a.nb - 1) && (a.rem > 0);
@@ -191,6 +185,28 @@ __device__ __forceinline__ void pair_sums(const YView& a, int64_t base, int lane
             ab += fabsf(x);
           }
         }
+    };
+    if constexpr (!NARROW) {
+      if (how[g]) whole();
+      else if (p < a.npairs) elements();
+    } else {
+      if (__builtin_amdgcn_ballot_w64(how[g] >= 2)) {
+        if (how[g]) {
+          const bool last = how[g] == 3;
+          const int wid = last ? (int)a.rem : (int)a.bs;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int sh = 8 * (q + 4 * j) + 8 - wid;
+            uint32_t ns[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ns[e] = last ? ns2[4 * j + e] : sg2[4 * j + e];
+            acc8<DT>(drop_low(v[g][j], sh < 0 ? 0 : sh < 8 ? sh : 8), ns, pl, sg, sq, ab);
+          }
+        }
+      } else if (how[g] == 1) {
+        whole();
+      }
+      if (how[g] == 0 && p < a.npairs) elements();
     }
     pl = quad_sum(pl); sg = quad_sum(sg); sq = quad_sum(sq); ab = quad_sum(ab);
     if (q == g) { my_pl = pl; my_sg = sg; my_sq = sq; my_ab = ab; }

@@ -816,10 +816,13 @@ __global__ __launch_bounds__(64 * NW, TRF == 4 ? 1 : 2) void rs_gemm_tall_kernel
   const uint32_t ct = tile % nct;
   const int64_t c0 = (int64_t)ct * TC;
   const bool do_xn = XNORM && ct == 0;
-  // the depth's segments dealt to the NW waves of every depth part in order, as evenly as they go
-  const uint32_t nseg = (uint32_t)(g.k / SD), slot = half * NW + (uint32_t)w, slots = NW * (uint32_t)g.splits;
-  const int seg0 = (int)(nseg * slot / slots);
-  const int per = (int)(nseg * (slot + 1) / slots) - seg0;      // segments of this wave (0: more waves than segments)
+  // the depth's segments dealt to the NW waves of every depth part in order, as evenly as they go: wave `slot` starts at
+  // segment floor(segments slot / slots)
+  const uint32_t slot = half * NW + (uint32_t)w;
+  const uint32_t share = (uint32_t)g.seg_share, rest = (uint32_t)g.seg_rest, slots = NW * (uint32_t)g.splits;
+  const int seg0 = (int)(share * slot + (rest ? rest * slot / slots : 0u));
+  // (0: more waves than segments)
+  const int per = (int)(share * (slot + 1) + (rest ? rest * (slot + 1) / slots : 0u)) - seg0;
   uint8_t* const abuf = smem + w * 2 * RT_SEGB;
   // LDS address of fragment i (rows 32 i + r) at step jj of a segment: the 16-bit depth piece 4 h + jj, or the
   // fp8 byte offset 64 (jj / 4) + 32 h + 8 (jj % 4) (its 16-byte chunk c, swizzled by the row, and half of it)
@@ -1275,6 +1278,9 @@ int sdc_rs_gemm_tall_launch(int dtype, GemmArgs g, int role, hipStream_t stream)
   if (g.short_rows < 0 || g.short_rows > (byte_a ? 1 : 2) || (g.short_rows && !byte_a && !g.XN))
     return SDC_EUNSUPPORTED;
   if (dtype == SDC_I8) g.short_rows = 1;                        // (int8: 64-row tiles only)
+  const int64_t slots = (g.short_rows && !byte_a ? 8 : RS_WAVES) * g.splits, nseg = g.k / kmul;
+  g.seg_share = (int)(nseg / slots);
+  g.seg_rest = (int)(nseg % slots);
   const int64_t tr = g.short_rows == 2 ? 32 : g.short_rows ? 64 : 32 * SDC_TALL_TRF;
   const int64_t rtiles = sdc_cdiv(g.m, tr) + (g.goffs ? g.ngroups : 0);
   if (g.xf_blocks < 0 || (g.xf_blocks && (g.goffs || dtype == SDC_FP8))) return SDC_EINVAL;

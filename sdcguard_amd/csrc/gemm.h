@@ -25,17 +25,19 @@ struct GemmArgs {
   // takes every depth slice of some row tiles (its rows' 128-byte lines stay in its L2 between the two stages that
   // read their halves: for a tall A read once, whose parts fit one L2 whole)
   int rows_per_xcd;
-  // (the tall-tile kernel) the grid's last xf_blocks workgroups run the x pass's finishing step for row blocks
-  // 0 .. xf_blocks - 1 instead of tiles: sdc_linear_check's row GEMM leaves CUs idle, and xfinish has no other use
-  // for them
-  XStageArgs xf;
-  int xf_blocks;
-  // (the tall-tile kernel) 1: 64-row tiles instead of 128, 2: 32-row tiles (16-bit A only), for a short A whose
-  // 128-row tiles would be mostly padding or leave most CUs idle
-  int short_rows;
   // sets of result slots that workgroup 0 clears for the scoring pass that follows (null: none)
   unsigned long long* slots;
   int slot_sets;
+  // (the tall-tile kernel) 1: 64-row tiles instead of 128, 2: 32-row tiles (16-bit A only), for a short A whose
+  // 128-row tiles would be mostly padding or leave most CUs idle
+  int short_rows;
+  // (the tall-tile kernel, set by its launcher) the depth's segments by the waves that share them: whole share and rest
+  int seg_share, seg_rest;
+  // (the tall-tile kernel) the grid's last xf_blocks workgroups run the x pass's finishing step for row blocks
+  // 0 .. xf_blocks - 1 instead of tiles: sdc_linear_check's row GEMM leaves CUs idle, and xfinish has no other use
+  // for them
+  int xf_blocks;
+  XStageArgs xf;
 };
 
 // E and XN for `batches` batches.

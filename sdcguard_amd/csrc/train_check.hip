@@ -726,7 +726,7 @@ __global__ __launch_bounds__(256) void grouped_score_kernel(TrainArgs a) {
     float pl, sg, sq, ab;
     pair_sums<DT, NARROW>(a.cv, base, lane, sg2, ns2, pl, sg, sq, ab);
     grp = group_of(offs, a.ngroups, r);
-    if (grp >= 0) train_pair<DT>(a, p, pl, sg, sq, ab, tb, grp, &pe);
+    if (grp >= 0) train_pair<DT, false>(a, p, pl, sg, sq, ab, tb, grp, &pe);
     const int64_t last = base + 63 < a.cv.npairs ? base + 63 : a.cv.npairs - 1;
     g0 = group_of(offs, a.ngroups, base / a.cv.nb);
     g1 = group_of(offs, a.ngroups, last / a.cv.nb);
