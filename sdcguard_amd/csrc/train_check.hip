@@ -798,11 +798,13 @@ Layout layout(int64_t batch_a, int64_t batch_b, int64_t m, int64_t k, int64_t n,
   L.off_col = o; o += al(batch_b * L.ncols * 3);
   L.off_bmax = o; o += al(batch_b * L.nb);
   L.off_bias = o; o += al(3 * L.nb);
-  L.off_parts = o; o += al((batch_b * 3 * L.ncols * L.kp + 1) / 2);      // 16-bit parts, two per float
   const int64_t k64 = sdc_cdiv(k, 64) * 64;
   if (grouped) L.fragb = k % TALL_K == 0 ? sdc_parts_fragments_bytes(L.ncols, k) : 0;
   else L.fragb = L.nbt == 1 ? sdc_parts_fragments_bytes(L.ncols, k64) : 0;
-  L.off_frag = o; o += al(batch_b * L.fragb / 4);
+  // the 16-bit parts, two per float: k-major or in fragment order, one or the other (check_with turns to the k-major ones
+  // where no GEMM took the fragments)
+  L.off_parts = L.off_frag = o;
+  o += std::max(al((batch_b * 3 * L.ncols * L.kp + 1) / 2), al(batch_b * L.fragb / 4));
   L.esplits = !L.fragb ? L.splits
                        : std::max<int64_t>(L.splits, grouped ? 2 : std::max(sdc_tall_plan(m, k64, L.ncols, true).splits,
                                                                             sdc_tall_plan(m, k64, L.ncols, false).splits));
@@ -1284,9 +1286,10 @@ __global__ __launch_bounds__(256) void pack_consts_kernel(PackArgs a) {
 
 }  // namespace
 
+// (the block sums and their statistics; the parts go to the caller's buffer)
 extern "C" int64_t sdc_layer_constants_workspace(int64_t n, int64_t k, int64_t bs) {
   if (n <= 0 || k <= 0 || bs <= 0) return 0;
-  return layout(1, 1, 1, k, n, bs).total * (int64_t)sizeof(float) + 256;
+  return layout(1, 1, 1, k, n, bs).off_parts * (int64_t)sizeof(float) + 256;
 }
 
 extern "C" int sdc_layer_constants(int dtype, const void* W, int64_t swn, int64_t n, int64_t k, int64_t bs,
@@ -1300,7 +1303,7 @@ extern "C" int sdc_layer_constants(int dtype, const void* W, int64_t swn, int64_
   if (!W || !sign_table || !parts || !consts_bias || !consts_plain) return SDC_EINVAL;
   const Layout L = layout(1, 1, 1, k, n, bs);
   if (parts_pitch != L.kp) return SDC_EINVAL;
-  if (!workspace || workspace_bytes < L.total * (int64_t)sizeof(float) + 256) return SDC_EWORKSPACE;
+  if (!workspace || workspace_bytes < L.off_parts * (int64_t)sizeof(float) + 256) return SDC_EWORKSPACE;
   float* ws = (float*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
   const float* s_full = sign_table + (bs - 1) * 128;
   const float* s_last = L.rem ? sign_table + (L.rem - 1) * 128 : s_full;

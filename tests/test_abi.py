@@ -67,3 +67,18 @@ def test_ctypes_signatures_take_as_many_arguments_as_the_header_declares():
     for name, n in counts.items():
         assert name in _lib.SIGNATURES, name
         assert len(_lib.SIGNATURES[name][1]) == n, (name, len(_lib.SIGNATURES[name][1]), n)
+
+
+@pytest.mark.parametrize("m,k,n", [(3, 3162, 7471), (354, 2192, 34), (1024, 1024, 50257), (4096, 4096, 14336), (8192, 8192, 50257)])
+def test_workspaces_hold_each_thing_once(m, k, n):
+    """The training check's scratch holds the block sums, one copy of their parts (k-major or in fragment order) and at
+    most the planes of its GEMMs; a layer's constants need the block sums and their statistics only."""
+    from sdcguard_amd import _lib
+    L = _lib.lib()
+    nb = -(-n // 128)
+    sums = 4 * (2 * nb * k + 5 * nb * -(-k // 64) + 12 * nb)
+    parts = max(6 * 2 * nb * (k + 7), L.sdc_parts_fragments_bytes(2 * nb, -(-k // 64) * 64))
+    slack = 16 * 256
+    assert L.sdc_layer_constants_workspace(n, k, 128) <= sums + slack
+    planes = 8 if m >= 512 else 32
+    assert L.sdc_matmul_check_workspace(1, 1, m, k, n, 128) <= sums + parts + 4 * planes * m * (2 * nb + 2) + slack
