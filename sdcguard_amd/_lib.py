@@ -127,11 +127,17 @@ def check(rc: int, what: str) -> None:
         raise HipLibraryError(f"{what}: {_NAMES.get(rc, 'error')} (status {rc}){extra}")
 
 
+# torch's own query of a device's current raw stream, where this torch has it: making the Stream object that
+# torch.cuda.current_stream returns takes 1.8 us, twice a check, of 24 us for a serving check's whole call
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _raw_stream(device: torch.device) -> int:
-    """The raw hipStream_t of the current stream of a device.  (torch's own query of it: making the Stream object that
-    torch.cuda.current_stream returns takes 1.8 us, twice a check, of 24 us for a serving check's whole call.)"""
+    """The raw hipStream_t of the current stream of a device."""
+    if _current_raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    return _current_raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def stream_of(t: torch.Tensor) -> int:

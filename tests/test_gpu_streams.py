@@ -138,3 +138,16 @@ def test_constants_of_inference_mode(k):
         check_static_impl(x, y, _elsewhere(cs.parts), *cs.tensors(False)[1:], state, 0, 6.0, 1e-30, scores_out=again)
     assert (z >= 0).all() and float(z.max()) < 6.0 and float((z - again).abs().max()) < 1e-2
     assert int(state[0, 2]) == 2
+
+
+@pytest.mark.parametrize("query", ["raw", "stream"])
+def test_current_stream_handle(query, monkeypatch):
+    """The handle of torch's raw query, and of the stream object where a torch has no such query."""
+    from sdcguard_amd import _lib
+    if query == "stream":
+        monkeypatch.setattr(_lib, "_current_raw_stream", None)
+    t, side = torch.zeros(1, device="cuda"), torch.cuda.Stream()
+    assert _lib.stream_of(t) == torch.cuda.current_stream().cuda_stream == torch.cuda.default_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert _lib.stream_of(t) == side.cuda_stream
+        assert _lib._raw_stream(torch.device("cuda")) == side.cuda_stream
