@@ -117,7 +117,7 @@ class QuantChecksums:
             bfrob = torch.empty(nb, dtype=torch.float32, device=dev)
             bcol = torch.empty(n, dtype=torch.float32, device=dev)
             ws = torch.empty(int(L.sdc_quant_constants_workspace(1, k, n)), dtype=torch.uint8, device=dev)
-            scales = None if sb is None else sb.double().reshape(n).contiguous()
+            scales = None if sb is None else sb.double().view(n).contiguous()
         _lib.check(L.sdc_quant_constants(0 if i8 else 1, B.data_ptr(), B.stride(0), B.stride(1), k, n, block,
                                          tab.data_ptr(), _lib.ptr(scales) or None, parts.data_ptr(),
                                          _lib.ptr(bfrob) or None, _lib.ptr(bcol) or None, _lib.ptr(ws) or None,

@@ -475,3 +475,15 @@ def test_constants_made_on_the_device(kind, k, n, layout, block):
     assert torch.allclose(c.bcol.cpu().double(), Bd.square().sum(0).sqrt(), rtol=2.0 ** -23, atol=0)
     frob = torch.stack([Bd[:, lo:lo + block].square().sum().sqrt() for lo in range(0, n, block)])
     assert torch.allclose(c.bfrob.cpu().double(), frob, rtol=2.0 ** -23, atol=0)
+
+
+def test_scales_of_another_shape():
+    """Scales that do not view as one per column are refused, on either path."""
+    from sdcguard_amd import modes
+    B = torch.randn(64, 32).to(torch.float8_e4m3fn)
+    for b in (B, B.cuda()):
+        for sb in (torch.ones(4, 8, device=b.device).t(), torch.ones(31, device=b.device)):
+            with pytest.raises(RuntimeError):
+                modes.QuantChecksums.make(b, sb)
+        for sb in (torch.ones(4, 8, device=b.device), torch.ones(64, device=b.device)[::2]):
+            assert modes.QuantChecksums.make(b, sb).n == 32
