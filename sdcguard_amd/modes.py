@@ -93,7 +93,9 @@ class QuantChecksums:
             return cls("int8", k, n, block, parts)
         if B.dtype == torch.float8_e4m3fn:
             Bs = B.double() if sb is None else B.double() * sb.double().view(1, n)
-            B2s = (Bs @ W).float()
+            # block by block, as sdc_quant_constants: a NaN or an infinite scale spoils its own block's sums only (0 x NaN)
+            B2s = torch.cat([Bs[:, lo:lo + block] @ W[lo:lo + block, 2 * b:2 * b + 2]
+                             for b, lo in enumerate(range(0, n, block))], 1).float()
             parts = _split3(B2s.t().contiguous())                  # (3, 2nb, k)
             nb = W.shape[1] // 2
             pad = nb * block - n

@@ -477,6 +477,37 @@ def test_constants_made_on_the_device(kind, k, n, layout, block):
     assert torch.allclose(c.bfrob.cpu().double(), frob, rtol=2.0 ** -23, atol=0)
 
 
+@pytest.mark.parametrize("where", ["cpu", "cuda"])
+def test_nonfinite_weights_and_scales(where):
+    """A NaN weight or an infinite scale (of a column that holds zeros too) spoils its own block's constants and
+    verdicts, and no other's, wherever the constants are made."""
+    from sdcguard_amd import modes
+    m, k, n = 70, 192, 500
+    g = torch.Generator().manual_seed(5)
+    A = torch.randn(m, k, generator=g).to(torch.float8_e4m3fn)
+    B = torch.randn(k, n, generator=g)
+    B[::2, 300] = 0.0
+    B[7, 130] = float("nan")
+    B = B.to(torch.float8_e4m3fn)
+    sb = torch.rand(n, generator=g) + 0.5
+    sb[300] = float("inf")
+    C = (A.double() @ (B.double() * sb.double())).float()
+    consts = modes.QuantChecksums.make(B.to(where), sb.to(where))
+    bad = torch.tensor([False, True, True, False])
+    sums = consts.parts.double().sum(0).view(4, 2, k).cpu()
+    assert torch.equal(torch.isfinite(sums).all(2).all(1), ~bad)
+    assert torch.isfinite(sums[1]).sum() == 2 * (k - 1) and torch.equal(torch.isfinite(consts.bfrob.cpu()), ~bad)
+    assert torch.equal(torch.isfinite(consts.bcol.cpu()).nonzero(as_tuple=True)[0],
+                       torch.tensor([j for j in range(n) if j not in (130, 300)]))
+    consts = modes.QuantChecksums("fp8", k, n, 128, consts.parts.cuda(), consts.bfrob.cuda(), consts.bcol.cuda())
+    z = torch.empty(m, 4, device="cuda")
+    row = modes.quant_zscores(A.cuda(), consts, C.cuda(), scores_out=z).result.tolist()
+    o = quant.fp8_judge(A.double().numpy(), B.double().numpy(), np.ones(m), sb.double().numpy(), C.double().numpy(),
+                        quant.patterns(1))
+    assert np.array_equal(np.isinf(z.cpu().numpy()), np.isinf(o["z"])) and row[2] == o["wrong_blocks"] == 2 * m
+    assert np.isinf(o["z"])[:, bad.numpy()].all() and not np.isinf(o["z"])[:, ~bad.numpy()].any()
+
+
 def test_scales_of_another_shape():
     """Scales that do not view as one per column are refused, on either path."""
     from sdcguard_amd import modes
