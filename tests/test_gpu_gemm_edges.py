@@ -85,3 +85,76 @@ def test_narrow_blocks(n, block, batch, dt):
     z = scores.cpu().numpy().reshape(-1)
     ok = z_close(z, o.z.reshape(-1), gemm_slack(o.csb, o.den).reshape(-1))
     assert ok.all(), (np.nonzero(~ok)[0][:5], z[~ok][:5], o.z.reshape(-1)[~ok][:5])
+
+
+def _scores_match(A, B, C, dt, **kw):
+    """Every score and the count of unjudged ones against the oracle's."""
+    from sdcguard_amd import matmul_zscores
+    m, n = C.shape
+    scores = torch.full((1, m, -(-n // 128), 2), -7.0, device="cuda")
+    row = matmul_zscores(A, B, C, scores_out=scores, **kw).result.tolist()
+    o = abft.zscores(*(t.float().cpu().numpy() for t in (A, B, C)), dtype=dt, seed=1, **kw)
+    z = scores.cpu().numpy().reshape(-1)
+    ok = z_close(z, o.z.reshape(-1), gemm_slack(o.csb, o.den).reshape(-1))
+    assert ok.all(), (np.nonzero(~ok)[0][:5], z[~ok][:5], o.z.reshape(-1)[~ok][:5])
+    assert row[2] == int((o.z < 0).sum())
+    return z.reshape(m, -1), o
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("m,k,n,la,lc", [(131, 65, 300, "odd", "rows"), (130, 64, 257, "rows", "odd"),
+                                         (257, 130, 513, "cols_odd", "cols"), (67, 5, 9, "rows", "rows"),
+                                         (37, 63, 130, "strided", "strided")])
+def test_nonfinite_at_the_edges(m, k, n, la, lc, bad, dt):
+    """NaN and infinities at the ends of rows, columns, narrow blocks and depth, in each operand: the pairs that hold
+    them get the oracle's verdict, and rows and blocks beside them are judged as without them."""
+    g = torch.Generator().manual_seed(m + k)
+    t = torch.bfloat16 if dt == "bf16" else torch.float16
+    A, B, C = _operand(m, k, la, g, t, 1.0), _operand(k, n, "rows", g, t, 0.1), _operand(m, n, lc, g, t, 1.0)
+    C.copy_((A.float() @ B.float()).to(t))
+    clean, _ = _scores_match(A, B, C, dt)
+    last = n - 1
+    for T, i, j in ((C, m - 1, last), (C, 0, 0), (C, m // 2, last - last % 128 - 1 if n > 128 else 0), (C, 3, last - last % 128),
+                    (A, m - 1, k - 1), (A, 0, k - 1), (A, m - 2, 0)):
+        kept = T[i, j].clone()
+        T[i, j] = bad
+        z, _ = _scores_match(A, B, C, dt)
+        others = torch.arange(m).numpy() != i
+        assert np.array_equal(z[others], clean[others])
+        T[i, j] = kept
+    for i, j in ((k - 1, last), (0, 0)):
+        kept = B[i, j].clone()
+        B[i, j] = bad
+        z, o = _scores_match(A, B, C, dt)
+        blocks = np.arange(z.shape[1]) // 2 != j // 128
+        assert np.array_equal(z[:, blocks], clean[:, blocks])
+        B[i, j] = kept
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("la", ["rows", "odd", "cols", "strided"])
+@pytest.mark.parametrize("lc", ["rows", "cols"])
+def test_many_planes(la, lc, dt):
+    """A deep product of few rows and columns: more depth parts than a scoring pass loads at once, for both ways of reading C."""
+    from sdcguard_amd import _lib
+    m, k, n = 300, 8256, 260
+    g = torch.Generator().manual_seed(9)
+    t = torch.bfloat16 if dt == "bf16" else torch.float16
+    A, B, C = _operand(m, k, la, g, t, 1.0), _operand(k, n, "rows", g, t, 0.02), _operand(m, n, lc, g, t, 1.0)
+    C.copy_((A.float() @ B.float()).to(t))
+    C[m - 1, n - 1] += 8.0
+    z, o = _scores_match(A, B, C, dt)
+    assert (z > 6).any()
+
+
+@pytest.mark.parametrize("dt,scale", [("fp16", 1e-4), ("fp16", 4e-4), ("bf16", 3e-10)])
+@pytest.mark.parametrize("n,lc", [(256, "rows"), (300, "rows"), (300, "odd"), (9, "rows"), (300, "cols"), (300, "strided")])
+def test_subnormal_outputs(n, lc, dt, scale):
+    """fp16 outputs below the normal range, and bf16 ones whose squares are below fp32's, keep their sums and norms."""
+    m, k = 70, 64
+    g = torch.Generator().manual_seed(n)
+    t = torch.bfloat16 if dt == "bf16" else torch.float16
+    A, B, C = _operand(m, k, "rows", g, t, scale), _operand(k, n, "rows", g, t, scale), _operand(m, n, lc, g, t, 1.0)
+    C.copy_((A.float() @ B.float()).to(t))
+    _scores_match(A, B, C, dt, abs_floor=1e-30)
