@@ -43,8 +43,9 @@ extern "C" {
  *     [scale0, scale1, bsum0, bsum1, b2n0, b2n1, b2max0, b2max1, bmax, bmax_bias, 0, 0]: three 16-byte loads
  *     per block instead of ten scattered ones; the separate arrays are still required.
  *   parts_frag (may be NULL; no counterpart in the reference): the parts in sdc_parts_fragments' order, 16-byte
- *     aligned, made once per layer: with them (k-contiguous 16-bit x, depth a multiple of 512) the expected side
- *     runs on the register-streamed tall-tile GEMM (two planes of E) instead of the staged one. */
+ *     aligned, made once per layer: with them (k-contiguous 16-bit x, rows 16-byte aligned, depth a multiple of 64)
+ *     the expected side runs on the register-streamed tall-tile GEMM (1 to 32 planes of E, by the shape) instead of the
+ *     staged one. */
 int64_t sdc_check_static_workspace(int64_t m, int64_t k, int64_t n, int64_t bs);
 int sdc_check_static(int dtype, const void* x, int64_t sxm, int64_t sxk, const void* y, int64_t sym, int64_t syn,
                      int64_t m, int64_t k, int64_t n, int64_t bs, const void* parts, int64_t spk, int64_t spc,
@@ -252,7 +253,8 @@ int sdc_digit_fragments(const void* parts, int64_t spc, int64_t N, int64_t k, vo
  *   kind 0 (int8): parts (2, 2 nb, k rounded up to even) int8, the block sums' base-128 digits; no sb.  (Every sum
  *     splits unless it is 16384: 128 entries of -128 under a pattern of -1 only, which the caller refuses.)
  *   kind 1 (fp8 e4m3): parts (3, 2 nb, k) bf16 of the scaled sums (sb: n float64 column scales, or NULL for 1), bfrob
- *     (nb) and bcol (n) fp32; ws: sdc_quant_constants_workspace(kind, k, n) bytes. */
+ *     (nb) and bcol (n) fp32; ws: sdc_quant_constants_workspace(kind, k, n) bytes.  A NaN in B or an infinite scale spoils
+ *     the sums and norms of its own block only. */
 int64_t sdc_quant_constants_workspace(int kind, int64_t k, int64_t n);
 int sdc_quant_constants(int kind, const void* B, int64_t sbk, int64_t sbn, int64_t k, int64_t n, int64_t block,
                         const float* sign_table, const double* sb, void* parts, float* bfrob, float* bcol, void* ws,

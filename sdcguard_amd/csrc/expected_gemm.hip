@@ -709,8 +709,9 @@ __global__ __launch_bounds__(64 * RS_WAVES, 1) void rs_gemm_kernel(GemmArgs g) {
 // ------------------------------------------------------------------------- register-streamed GEMM, tall tiles
 // The same loop with 128 rows of A per wave: each B fragment loaded from L2 meets twice the rows, so a workgroup
 // moves 36% fewer bytes through the vector memory path per MFMA (1.25 MB instead of 2 MB for the same 64 x 64 x
-// 4096 worth of products).  The workgroup tile is 128 x 64 over half the depth; the two halves are separate
-// workgroups, each writing its own plane of E (plane h = depth half h), which the scoring pass adds in half order.
+// 4096 worth of products).  The workgroup tile is 128 x 64 (a short A: 64 x 64 or 32 x 64) over one of g.splits depth
+// parts; the parts are separate workgroups, each writing its own plane of E (plane h = part h), which the scoring pass
+// adds in part order.
 // A's ring per wave is two 16 KB segments (128 rows x 128 bytes; 128 KB for the 4 waves), the next segment loading
 // while the current one is read.  A segment is 64 depths of a 16-bit A, or 128 of an fp8 A (AT = 1: one byte per
 // element, widened exactly to bf16 after the LDS read; the MFMAs are bf16), so 4 or 8 steps of 16 depths.  Per step
@@ -719,8 +720,9 @@ __global__ __launch_bounds__(64 * RS_WAVES, 1) void rs_gemm_kernel(GemmArgs g) {
 // a segment, those after the segment's last A piece are the 6 B loads of one step: the wait is
 // vmcnt((RB - 1) (APS + 6)) inside a segment and vmcnt(6) at its first step.
 // XN: the workgroups of the first column tile also add up |a_row|_2^2 and |a_row|_1 of their rows (from the A
-// fragments, over their depth half) into plane `half` of g.XN ([half][2][m]).
-// XCD order: XCDs 0-3 take depth half 0 and 4-7 half 1 (each XCD's L2 holds its half of B), row tiles in order.
+// fragments, over their depth part) into plane `half` of g.XN ([part][2][m]; `half` is the part's number throughout).
+// XCD order: XCD x takes the x-th eighth of the (part, row tile, column tile) list where the grid is whole eighths, so its
+// L2 holds the parts of B it needs: with two parts, XCDs 0-3 the first and 4-7 the second.
 #ifndef SDC_TALL_TRF
 #define SDC_TALL_TRF 4
 #endif
@@ -1047,7 +1049,7 @@ __global__ __launch_bounds__(64 * NW, TRF == 4 ? 1 : 2) void rs_gemm_tall_kernel
   }
   if constexpr (XNORM) {
     if (do_xn) {
-      // the two depth halves of a row (lanes r, r + 32), then the four waves' depth quarters in LDS, in wave order
+      // the two lanes of a row (r, r + 32: other depths of each step), then the waves' depth shares in LDS, in wave order
 #pragma unroll
       for (int i = 0; i < TRF; ++i) {
         xsq[i] += __shfl_xor(xsq[i], 32, 64);

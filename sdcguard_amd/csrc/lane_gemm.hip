@@ -14,8 +14,8 @@
 //     rows an instruction, then through the wave's own 16 KB of LDS (16-byte piece p of row r at position p ^ (r % 8)).
 //     Loads of a row a lane touched 64 lines an instruction, each line again by seven more.
 // Bound by the loads in flight (16 KB a wave) and the matrix cores.  Measured on MI355X: dy^T 14336 x 4096 (64 columns)
-// 34 us, from 125 us with the staged GEMM's element loads; with 12 columns, dy 1024 x 50257 38 us (from 66 us with loads
-// straight into the operands' registers and 64-column tiles) and dy^T 50257 x 1024 41 us (from 69 us, with
+// 34-36 us, from 125 us with the staged GEMM's element loads; with 12 columns, dy 1024 x 50257 37 us (from 66 us with loads
+// straight into the operands' registers and 64-column tiles) and dy^T 50257 x 1024 40 us (from 69 us, with
 // every row tile's last segment element by element).
 #include "blocksums.h"
 #include "common.h"

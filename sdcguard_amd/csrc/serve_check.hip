@@ -207,7 +207,7 @@ __device__ __forceinline__ void report_wg(const ScoreArgs& a, LaneBest best) {
 
 // v1 (one launch after the GEMM): sums and scores in the same pass over y.  Each wave walks tiles of 64 pairs
 // with a grid stride and keeps its worst key; the workgroup reports once at the end.  A tile's expected sums (NS
-// planes: 2 from the tall-tile GEMM) are loaded before its outputs, so both arrive in one round trip.
+// planes) are loaded before its outputs, so both arrive in one round trip; further planes are added in a loop (GEN).
 // GEN: y has blocks narrower than 128, or the GEMM more than NS planes.
 template <int DT, int NS, bool GEN>
 __global__ __launch_bounds__(256) void serve_fused_kernel(ScoreArgs a) {

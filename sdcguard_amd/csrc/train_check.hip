@@ -2,13 +2,16 @@
 //
 // Reference: checksum.py:435-530 (`_zscores`: the arithmetic), :349-383 (`_complete_score`, `_judge_nonfinite`:
 // the Inf/NaN rules with unjudged checksums scoring -1), _group.py:386-746 (the device version it replaces: B-side
-// stage, comparison, worst-z search).  Four launches, no host synchronisation:
+// stage, comparison, worst-z search).  Four launches (five for fp16, and where the parts are k-major), no host
+// synchronisation:
 //   1. b_stage: the plain and signed block sums of every row of B (B2, fp32, stored transposed so the GEMM reads
 //      depth-contiguous columns) and, per 64-row slice, partial sums of squares / maxima of B2's columns and the
 //      largest |B| of every block;
-//   2. b_finish: those partials added up (|checksum column|_2, its largest entry, the per-column power of two that
-//      keeps fp16 parts in range, the block's largest |B|) and the bias vector's block sums;
-//   3. split + expected_gemm (expected_gemm.hip): B2 as three parts, E = A @ B2 on MFMA, plus A's row norms;
+//   2. those partials added up (|checksum column|_2, its largest entry, the per-column power of two that keeps fp16
+//      parts in range, the block's largest |B|), the bias vector's block sums, and B2 as three parts: finish_frag, in
+//      fragment order (fp16: b_finish for the scales first); or b_finish and split, k-major, for batches and other strides of A;
+//   3. E = A @ B2 on MFMA, plus A's row norms: the tall-tile GEMM (rows in whole lines), lane_gemm (rows at any
+//      address, or contiguous across each other), else the staged GEMM;
 //   4. train_score: one persistent pass over C scoring every (batch, row, block) pair, worst key and unjudged count
 //      into the check's result row with atomics.
 #include <type_traits>
